@@ -18,7 +18,10 @@
 namespace musc {
 namespace rscin {
 
-constexpr int kThreads = 256;
+constexpr int kThreads = 1024;   // 16 waves share a row's n similarities
+constexpr int kWaves = kThreads / kWave;
+constexpr int kRowsAtOnce = 4;   // similarities a wave forms together
+constexpr int kSteps = 3;        // 64-vector steps whose loads are in flight together
 constexpr int kMaxN = 4096;
 constexpr int kMaxK = 16;
 
@@ -30,11 +33,34 @@ struct KList {
   int n;
 };
 
+// wave_sum of several values, their exchanges in flight together.
+template <int kCount>
+__device__ inline void wave_sums(double (&v)[kCount]) {
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    double t[kCount];
+#pragma unroll
+    for (int r = 0; r < kCount; ++r) t[r] = __shfl_xor(v[r], off, kWave);
+#pragma unroll
+    for (int r = 0; r < kCount; ++r) v[r] += t[r];
+  }
+}
+
+// Latency-bound: n workgroups of a few microseconds of work each.  A wave forms four
+// similarities at a time, all loads of up to 768 channels in flight together, where one
+// row at a time waited for memory once per 64 channels; 16 waves share the row; each
+// entry's rank is counted once for all of k_list, by several lanes.  N = 83, d = 768,
+// k = 1, 2, 3, right after the map kernel: 12.1 us, against 88.7 us with 4 waves, one
+// similarity at a time, scalar loads and a rank count per k (N = 1000: 0.50 against
+// 1.08 ms).
+template <int kVec>  // floats per load: 4 when every row is 16-byte aligned, else 1
 __global__ __launch_bounds__(kThreads) void rscin_kernel(const float* __restrict__ x, const double* __restrict__ raw,
-                                                         int n, int d, KList ks, float* __restrict__ out) {
+                                                         int n, int d, int share, KList ks, float* __restrict__ out) {
+  typedef float vec __attribute__((ext_vector_type(kVec)));
   extern __shared__ double w[];  // n similarities of row i
-  __shared__ double red[2][kThreads / kWave];
-  __shared__ double s_min, s_max;
+  __shared__ double s_range[2][kWaves];
+  __shared__ double s_part[kMaxK][2][kWaves];
+  __shared__ double s_ratio[kMaxK];
   const int i = blockIdx.x, tid = threadIdx.x;
   const int wave = tid / kWave, lane = tid % kWave;
   // min / max of the raw scores
@@ -49,65 +75,108 @@ __global__ __launch_bounds__(kThreads) void rscin_kernel(const float* __restrict
     mx = nmax(mx, __shfl_xor(mx, off, kWave));
   }
   if (lane == 0) {
-    red[0][wave] = mn;
-    red[1][wave] = mx;
+    s_range[0][wave] = mn;
+    s_range[1][wave] = mx;
+  }
+  // similarities W[i][j] = x_i . x_j (fp64 accumulation of the fp32 tokens): the loads of
+  // kSteps steps of 64 vectors, of this row and of kRowsAtOnce others, before the first use
+  const vec* xi = reinterpret_cast<const vec*>(x + (long long)i * d);
+  const int dv = d / kVec;
+  for (int j0 = wave * kRowsAtOnce; j0 < n; j0 += kWaves * kRowsAtOnce) {
+    const vec* xj[kRowsAtOnce];
+    double acc[kRowsAtOnce];
+#pragma unroll
+    for (int r = 0; r < kRowsAtOnce; ++r) {
+      xj[r] = reinterpret_cast<const vec*>(x + (long long)min(j0 + r, n - 1) * d);
+      acc[r] = 0.0;
+    }
+    for (int c0 = 0; c0 < dv; c0 += kSteps * kWave) {
+      vec a[kSteps], b[kSteps][kRowsAtOnce];
+#pragma unroll
+      for (int u = 0; u < kSteps; ++u) {
+        const int c = c0 + u * kWave + lane;
+        const bool ok = c < dv;  // vectors past the row add 0 x 0
+        const int cc = ok ? c : dv - 1;
+        a[u] = xi[cc];
+#pragma unroll
+        for (int r = 0; r < kRowsAtOnce; ++r) b[u][r] = xj[r][cc];
+        if (!ok) {
+          a[u] = vec{};
+#pragma unroll
+          for (int r = 0; r < kRowsAtOnce; ++r) b[u][r] = vec{};
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kSteps; ++u)
+#pragma unroll
+        for (int e = 0; e < kVec; ++e)
+#pragma unroll
+          for (int r = 0; r < kRowsAtOnce; ++r) acc[r] = fma((double)a[u][e], (double)b[u][r][e], acc[r]);
+    }
+    wave_sums(acc);
+#pragma unroll
+    for (int r = 0; r < kRowsAtOnce; ++r)
+      if (lane == 0 && j0 + r < n) w[j0 + r] = acc[r];
+  }
+  __syncthreads();
+  double lo = s_range[0][0], hi = s_range[1][0];
+#pragma unroll
+  for (int q = 1; q < kWaves; ++q) {
+    lo = nmin(lo, s_range[0][q]);
+    hi = nmax(hi, s_range[1][q]);
+  }
+  const double span = hi - lo;
+  double num[kMaxK], den[kMaxK];
+#pragma unroll
+  for (int q = 0; q < kMaxK; ++q) num[q] = den[q] = 0.0;
+  // an entry's rank is counted by `share` neighbouring lanes, each over every share-th entry
+  for (int t0 = 0; t0 < n * share; t0 += kThreads) {
+    const int j = (t0 + tid) / share, m0 = (t0 + tid) % share;
+    const bool own = j < n && m0 == 0;
+    const double v = w[min(j, n - 1)];
+    int rank = 0;  // entries strictly before j in descending order
+#pragma unroll 4
+    for (int m = m0; m < n; m += share) {
+      const double u = w[m];
+      rank += (u > v) | ((u == v) & (m < j));
+    }
+    for (int off = share / 2; off >= 1; off >>= 1) rank += __shfl_xor(rank, off, kWave);
+    if (own) {
+      const double s01 = (double)(float)((raw[j] - lo) / span);
+#pragma unroll
+      for (int q = 0; q < kMaxK; ++q)
+        if (q < ks.n && rank < ks.k[q]) {
+          num[q] += v * s01;
+          den[q] += v;
+        }
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < kMaxK; ++q)
+    if (q < ks.n) {
+      double part[2] = {num[q], den[q]};
+      if (wave * kWave < n * share) wave_sums(part);  // waves past the last entry hold zeros
+      if (lane == 0) {
+        s_part[q][0][wave] = part[0];
+        s_part[q][1][wave] = part[1];
+      }
+    }
+  __syncthreads();
+  if (tid < ks.n) {
+    double a = 0.0, b = 0.0;
+#pragma unroll
+    for (int r = 0; r < kWaves; ++r) {
+      a += s_part[tid][0][r];
+      b += s_part[tid][1][r];
+    }
+    s_ratio[tid] = a / b;
   }
   __syncthreads();
   if (tid == 0) {
-    double a = red[0][0], b = red[1][0];
-    for (int q = 1; q < kThreads / kWave; ++q) {
-      a = nmin(a, red[0][q]);
-      b = nmax(b, red[1][q]);
-    }
-    s_min = a;
-    s_max = b;
+    double total = 0.0;
+    for (int q = 0; q < ks.n; ++q) total += s_ratio[q];
+    out[i] = (float)(total / ks.n);
   }
-  // similarities W[i][j] = x_i . x_j (fp64 accumulation of the fp32 tokens)
-  const float* xi = x + (long long)i * d;
-  for (int j = wave; j < n; j += kThreads / kWave) {
-    const float* xj = x + (long long)j * d;
-    double acc = 0.0;
-    for (int c = lane; c < d; c += kWave) acc = fma((double)xi[c], (double)xj[c], acc);
-    acc = wave_sum(acc);
-    if (lane == 0) w[j] = acc;
-  }
-  __syncthreads();
-  const double lo = s_min, span = s_max - s_min;
-  double total = 0.0;
-  for (int q = 0; q < ks.n; ++q) {
-    const int k = ks.k[q];
-    double num = 0.0, den = 0.0;
-    for (int j = tid; j < n; j += kThreads) {
-      const double v = w[j];
-      int rank = 0;  // entries strictly before j in descending order
-      for (int m = 0; m < n; ++m) {
-        const double u = w[m];
-        rank += (u > v) || (u == v && m < j);
-      }
-      if (rank < k) {
-        const float s01 = (float)((raw[j] - lo) / span);
-        num += v * (double)s01;
-        den += v;
-      }
-    }
-    num = wave_sum(num);
-    den = wave_sum(den);
-    __syncthreads();
-    if (lane == 0) {
-      red[0][wave] = num;
-      red[1][wave] = den;
-    }
-    __syncthreads();
-    if (tid == 0) {
-      double a = 0.0, b = 0.0;
-      for (int r = 0; r < kThreads / kWave; ++r) {
-        a += red[0][r];
-        b += red[1][r];
-      }
-      total += a / b;
-    }
-  }
-  if (tid == 0) out[i] = (float)(total / ks.n);
 }
 
 }  // namespace rscin
@@ -125,7 +194,10 @@ extern "C" int musc_rscin_f32(const float* cls_tokens, const double* image_score
     if (k_list[q] < 1 || k_list[q] > n) return MUSC_ERR_INVALID_ARG;
     ks.k[q] = k_list[q];
   }
-  hipLaunchKernelGGL(rscin::rscin_kernel, dim3(n), dim3(rscin::kThreads), (size_t)n * sizeof(double), stream,
-                     cls_tokens, image_scores, n, d, ks, out);
+  int share = 1;  // lanes per entry of the rank count
+  while (share < 16 && n * share * 2 <= rscin::kThreads) share *= 2;
+  const bool vec4 = d % 4 == 0 && (reinterpret_cast<uintptr_t>(cls_tokens) & 15) == 0;
+  hipLaunchKernelGGL((vec4 ? rscin::rscin_kernel<4> : rscin::rscin_kernel<1>), dim3(n), dim3(rscin::kThreads),
+                     (size_t)n * sizeof(double), stream, cls_tokens, image_scores, n, d, share, ks, out);
   return check_launch();
 }

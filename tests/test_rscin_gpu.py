@@ -28,3 +28,27 @@ def test_passthrough(device):
     raw = np.arange(5.0)
     assert RsCIN(raw, None, [1]) is raw
     assert RsCIN(raw, [np.ones(4, np.float32)] * 5, [0, 1]) is raw
+
+
+@pytest.mark.parametrize('n,d', [(1, 4), (2, 3), (63, 772), (64, 769), (65, 768), (128, 1024), (129, 5), (512, 8),
+                                 (513, 12), (1025, 7)])
+@pytest.mark.parametrize('offset', [0, 1])
+def test_row_widths_and_pool_sizes(device, n, d, offset):
+    # widths with and without 16-byte rows (offset 1: an unaligned view of aligned rows) and pools
+    # at the sizes where the lanes per ranked entry change, against the float64 definition.  The
+    # kernel rounds the normalised scores (<= 1) and the result to fp32: 2 x 2^-25 in all, the
+    # weights being positive (a shared mean keeps every similarity positive)
+    rng = np.random.default_rng(n * 100 + d)
+    cls = (rng.standard_normal((n, d)) * 0.3 + 1.0).astype(np.float32)
+    cls /= np.linalg.norm(cls, axis=1, keepdims=True)
+    raw = rng.random(n) + np.arange(n) * 1e-3
+    flat = torch.zeros(n * d + offset, device=device)
+    flat[offset:] = torch.from_numpy(cls).reshape(-1).to(device)
+    ks = [k for k in (1, 3, 16) if k <= n]
+    if n == 1:
+        raw = np.array([0.5])
+    got = RsCIN(torch.from_numpy(raw).to(device), flat[offset:].view(n, d), ks).cpu().numpy()
+    if n == 1:                       # one score: 0 / 0 in the min-max normalisation
+        assert np.isnan(got).all()
+        return
+    np.testing.assert_allclose(got, orc.rscin_bruteforce_f64(raw, cls, ks), rtol=0, atol=1.2e-7)
