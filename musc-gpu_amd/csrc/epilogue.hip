@@ -5,32 +5,39 @@
 // mean over radii, view (N, 1, side, side), F.interpolate(size=S, bilinear,
 // align_corners=True), image score = max of each S x S map.
 //
-// One workgroup per (image, band of output rows: kRows when upsampling, fewer when a
-// strong downsampling would make kRows rows span more than kMaxGridRows grid rows,
-// down to one).  A band touches at most a few grid rows, so the workgroup averages
-// only those rows of the n_radii * n_layers score maps into LDS, then writes its
-// band of S-pixel rows (coalesced
-// float64 rows) and merges its band maximum into image_scores with a 64-bit
+// One workgroup per (image, band of output rows: up to kRows, fewer when the bands
+// would not fill the chip or a strong downsampling would make them span more than
+// kMaxGridRows grid rows).  A band touches a few grid rows, so the workgroup averages
+// only those rows of the n_radii * n_layers score maps into LDS.  Thread t owns output
+// column t (t + blockDim.x, ...) and walks down the band: the horizontal
+// interpolants of the two grid rows around an output row change only when the output
+// row passes a grid row, so a pixel costs the vertical interpolation and one store of a
+// whole coalesced row.  The band maximum is merged into image_scores with a 64-bit
 // atomicMax on the bit pattern (all scores are non-negative distances, whose
 // IEEE bits order like the values).  The maximum propagates NaN, as numpy's max
 // at models/musc.py:288 does: NaN bit patterns (either sign) compare above every
 // non-negative number as unsigned integers, so the atomic keeps them too.
+//
+// Bound by the float64 map writes: N = 83, 3 x 4 maps, 37 -> 518 (178 MB written, 11 MB
+// read) in 36.6 us = 5.2 TB/s, the rate of a large copy; 62.5 us when every pixel formed
+// its own coordinates and both horizontal interpolants in 8-row bands.
 #include "common.hpp"
 
 namespace musc {
 namespace epi {
 
-constexpr int kRows = 8;           // output rows per band at most
-constexpr int kThreads = 256;
+constexpr int kRows = 32;          // output rows per band at most
+constexpr int kMaxThreads = 1024;
 constexpr int kMaxSide = 128;
-constexpr int kMaxGridRows = 16;  // grid rows one band may touch
+constexpr int kMaxGridRows = 16;   // grid rows one band may touch
+constexpr int kFillBlocks = 256;   // workgroups wanted before bands grow (one per CU)
 
 __device__ inline double nmax(double a, double b) { return __builtin_elementwise_maximum(a, b); }
 
-__global__ __launch_bounds__(kThreads) void maps_kernel(const double* __restrict__ scores, int n_radii, int n_layers,
-                                                        int n, int side, int out_size, int rows,
-                                                        double* __restrict__ maps,
-                                                        unsigned long long* __restrict__ image_bits) {
+__global__ __launch_bounds__(kMaxThreads) void maps_kernel(const double* __restrict__ scores, int n_radii,
+                                                           int n_layers, int n, int side, int out_size, int rows,
+                                                           double* __restrict__ maps,
+                                                           unsigned long long* __restrict__ image_bits) {
   const int bands = (out_size + rows - 1) / rows;
   const int img = blockIdx.x / bands, band = blockIdx.x % bands;
   const int y0 = band * rows;
@@ -44,6 +51,8 @@ __global__ __launch_bounds__(kThreads) void maps_kernel(const double* __restrict
   const int ng = g1 - g0 + 1;
 
   __shared__ double avg[kMaxGridRows][kMaxSide];
+  __shared__ double s_lh1[kRows];
+  __shared__ int s_h0[kRows];
   for (int t = threadIdx.x; t < ng * side; t += blockDim.x) {
     const int gr = g0 + t / side, gc = t % side;
     const long long pix = (long long)gr * side + gc;
@@ -55,28 +64,46 @@ __global__ __launch_bounds__(kThreads) void maps_kernel(const double* __restrict
     }
     avg[t / side][gc] = rsum / (double)n_radii;
   }
+  if (threadIdx.x < y1 - y0) {
+    const double sy = scale * (y0 + (int)threadIdx.x);
+    const int h0 = (int)sy;
+    s_h0[threadIdx.x] = h0;
+    s_lh1[threadIdx.x] = sy - h0;
+  }
   __syncthreads();
 
   double vmax = 0.0;
-  const int pixels = (y1 - y0) * out_size;
-  for (int t = threadIdx.x; t < pixels; t += blockDim.x) {
-    const int y = y0 + t / out_size, x = t % out_size;
-    const double sy = scale * y, sx = scale * x;
-    const int h0 = (int)sy, w0 = (int)sx;
-    const int h1 = h0 < side - 1 ? h0 + 1 : h0;
+  for (int x = threadIdx.x; x < out_size; x += blockDim.x) {
+    const double sx = scale * x;
+    const int w0 = (int)sx;
     const int w1 = w0 < side - 1 ? w0 + 1 : w0;
-    const double lh1 = sy - h0, lh0 = 1.0 - lh1;
     const double lw1 = sx - w0, lw0 = 1.0 - lw1;
-    const double* r0 = avg[h0 - g0];
-    const double* r1 = avg[h1 - g0];
-    const double v = lh0 * (lw0 * r0[w0] + lw1 * r0[w1]) + lh1 * (lw0 * r1[w0] + lw1 * r1[w1]);
-    if (maps) maps[((long long)img * out_size + y) * out_size + x] = v;
-    vmax = nmax(vmax, v);
+    auto across = [&](int g) { return lw0 * avg[g - g0][w0] + lw1 * avg[g - g0][w1]; };
+    double* dst = maps ? maps + ((long long)img * out_size + y0) * out_size + x : nullptr;
+    int h = s_h0[0];                      // grid row of `top`; the same in every thread
+    double top = across(h), bottom = across(min(h + 1, side - 1));
+    int next_h0 = h;                      // the next output row's table entries, read one row ahead
+    double next_lh1 = s_lh1[0];
+    for (int y = 0; y < y1 - y0; ++y) {
+      const int h0 = next_h0;
+      const double lh1 = next_lh1, lh0 = 1.0 - lh1;
+      const int yn = min(y + 1, y1 - y0 - 1);
+      next_h0 = s_h0[yn];
+      next_lh1 = s_lh1[yn];
+      if (h0 != h) {
+        top = h0 == h + 1 ? bottom : across(h0);
+        bottom = across(min(h0 + 1, side - 1));
+        h = h0;
+      }
+      const double v = lh0 * top + lh1 * bottom;
+      if (dst) dst[(long long)y * out_size] = v;
+      vmax = nmax(vmax, v);
+    }
   }
   if (image_bits) {
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) vmax = nmax(vmax, __shfl_xor(vmax, off, kWave));
-    __shared__ double wmax[kThreads / kWave];
+    __shared__ double wmax[kMaxThreads / kWave];
     const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
     if (lane == 0) wmax[wave] = vmax;
     __syncthreads();
@@ -104,11 +131,19 @@ extern "C" int musc_maps_f64(const double* scores, int n_radii, int n_layers, in
   const double scale = out_size > 1 ? (double)(side - 1) / (double)(out_size - 1) : 0.0;
   int rows = epi::kRows;
   while (rows > 1 && (int)(scale * (rows - 1)) + 3 > epi::kMaxGridRows) --rows;
+  // 32-row bands repeat less of the averaging of the grid rows shared with their
+  // neighbours; 16-row bands only where 32 would leave CUs idle (3 x 4 maps, 37 -> 518, by
+  // N, 16 against 32 rows: N = 8 12.0 / 12.8 us, 16 15.9 / 15.7, 83 42.5 / 37.8)
+  if (rows > 16 && (long long)n * ((out_size + rows - 1) / rows) < epi::kFillBlocks) rows = 16;
+  // a handful of small maps: the walk down a band is all the time there is
+  if (rows > 8 && (long long)n * ((out_size + rows - 1) / rows) < epi::kFillBlocks / 4) rows = 8;
   const int bands = (out_size + rows - 1) / rows;
+  // a column per thread; at least four waves for the averaging
+  const int threads = min(max((out_size + kWave - 1) / kWave * kWave, 4 * kWave), epi::kMaxThreads);
   if ((long long)n * bands > 0x7fffffffLL) return MUSC_ERR_UNSUPPORTED;
   unsigned long long* bits = reinterpret_cast<unsigned long long*>(image_scores);
   if (bits) launch_fill_u32(reinterpret_cast<uint32_t*>(bits), (size_t)n * 2, 0u, stream);
-  hipLaunchKernelGGL(epi::maps_kernel, dim3((unsigned)(n * bands)), dim3(epi::kThreads), 0, stream, scores, n_radii,
+  hipLaunchKernelGGL(epi::maps_kernel, dim3((unsigned)(n * bands)), dim3(threads), 0, stream, scores, n_radii,
                      n_layers, n, side, out_size, rows, maps, bits);
   return check_launch();
 }

@@ -44,3 +44,15 @@ def test_degenerate_and_other_sizes(device, p, size):
     mean = raw.mean(axis=(0, 1)).reshape(4, side, side)
     brute = np.stack([oe.bilinear_align_corners_f64(m, size) for m in mean])
     np.testing.assert_allclose(maps[:, 0].cpu().numpy(), brute, rtol=0, atol=1e-12)
+
+
+@pytest.mark.parametrize('n,side,size', [(2, 37, 518), (35, 37, 518), (62, 37, 518), (40, 28, 517), (1, 5, 1030),
+                                         (33, 128, 1025), (3, 100, 33), (70, 2, 500), (64, 1, 512)])
+def test_band_heights_and_wide_rows(device, n, side, size):
+    # 8-, 16- and 32-row bands, rows wider than a workgroup, bands cut by the last row, downsampling
+    rng = np.random.default_rng(n * 1000 + size)
+    raw = rng.random((1, 2, n, side * side))
+    maps, img = _epilogue_hip.maps_and_scores(torch.from_numpy(raw).to(device), size)
+    ref_maps, ref_img = oe.maps_and_scores([[torch.from_numpy(raw[0, l]) for l in range(2)]], size)
+    np.testing.assert_allclose(maps.cpu().numpy(), ref_maps.numpy(), rtol=0, atol=1e-12)
+    np.testing.assert_allclose(img.cpu().numpy(), ref_img.numpy(), rtol=0, atol=1e-12)
