@@ -6,8 +6,7 @@
 // fused row softmax of models/modules/_attention_gpu.py:41-81 (fp32 max/sum,
 // fp16 storage).
 //
-// Layout trick: each wave computes S^T = K Q^T on fp32 MFMA
-// (v_mfma_f32_32x32x2f32) so that a lane owns ONE query (lane % 32) and 16 of the
+// Layout trick: each wave computes S^T = K Q^T on MFMA so that a lane owns ONE query (lane % 32) and 16 of the
 // 32 keys of a block in registers.  The row max / sum of the online softmax are
 // then in-register reductions plus one cross-half exchange, the rescale of the
 // running output is a per-lane scalar, and the probabilities already sit in the
@@ -111,21 +110,16 @@ __device__ inline void store_kv_row(float* __restrict__ Ks, float* __restrict__ 
   Vt[(d4 + 3) * VPITCH + key] = vv.w;
 }
 
-// The fp32 kernel runs one 12-wave workgroup (384 queries, 3 waves per SIMD) per CU
-// rather than three 4-wave ones: the wave arbiter favours the oldest waves, so of three
-// workgroups sharing a CU one finishes first and the last runs its final blocks alone,
-// with too few waves to keep the MFMA pipe busy; the barrier keeps 12 waves in step.
+// One 384-query tile in fp32 MFMA throughout: the products as they are, no scaling.
+// attn_fwd_kernel runs a tile here when its inputs do not fit the fp16 split.
 constexpr int WAVES32 = 12;
-__global__ __launch_bounds__(WAVES32 * kWave, 1) void attn_fwd_kernel(const float* __restrict__ qg,
-                                                                 const float* __restrict__ kg,
-                                                                 const float* __restrict__ vg,
-                                                                 float* __restrict__ og, int t, float scale_log2,
-                                                                 HeadLayout in, HeadLayout out, int nbh) {
-  __shared__ __attribute__((aligned(16))) float Ks[2][KB * KPITCH];
-  __shared__ __attribute__((aligned(16))) float Vt[2][D * VPITCH];
-
-  const int2 unit = fwd_unit<QW * WAVES32>(t, nbh);
-  if (unit.x < 0) return;
+constexpr int kF32Smem = (2 * KB * KPITCH + 2 * D * VPITCH) * 4;
+__device__ __forceinline__ void attend_tile_f32(float* smem, const float* __restrict__ qg,
+                                                const float* __restrict__ kg, const float* __restrict__ vg,
+                                                float* __restrict__ og, int t, float scale_log2,
+                                                const HeadLayout in, const HeadLayout out, int2 unit) {
+  float* const Ks0 = smem;  // two buffers of KB * KPITCH, then two of D * VPITCH
+  float* const Vt0 = smem + 2 * KB * KPITCH;
   const int bh = unit.x;
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
   const int lq = lane & 31, lh = lane >> 5;
@@ -184,7 +178,7 @@ __global__ __launch_bounds__(WAVES32 * kWave, 1) void attn_fwd_kernel(const floa
   for (int kb = 0; kb < nkb; ++kb) {
     const int buf = kb & 1;
     if (stager) {
-      store_kv_row(Ks[buf], Vt[buf], i0, k0, v0);
+      store_kv_row(Ks0 + buf * KB * KPITCH, Vt0 + buf * D * VPITCH, i0, k0, v0);
       // the block after the last is loaded again as the last block (never stored)
       const int nb = min(kb + 1, nkb - 1);
       const __amdgpu_buffer_rsrc_t rk = block_rsrc(kg, nb), rv = block_rsrc(vg, nb);
@@ -198,7 +192,7 @@ __global__ __launch_bounds__(WAVES32 * kWave, 1) void attn_fwd_kernel(const floa
     floatx16 s;
 #pragma unroll
     for (int v = 0; v < 16; ++v) s[v] = 0.f;
-    const float* krow = &Ks[buf][lq * KPITCH + 4 * lh];
+    const float* krow = Ks0 + buf * KB * KPITCH + lq * KPITCH + 4 * lh;
 #pragma unroll
     for (int ss = 0; ss < 8; ++ss) {
       const float4 a = *reinterpret_cast<const float4*>(krow + 8 * ss);
@@ -217,7 +211,7 @@ __global__ __launch_bounds__(WAVES32 * kWave, 1) void attn_fwd_kernel(const floa
 #pragma unroll
     for (int v = 1; v < 16; ++v) bmax = fmaxf(bmax, s[v]);
     bmax = halves_max(bmax);
-    // lazy rescaling, as in the fp16 kernel: the running maximum moves only past kLazyLog2
+    // lazy rescaling: the running maximum moves only past kLazyLog2
     if (!__all(bmax <= m + kLazyLog2)) {
       const float mnew = fmaxf(m, bmax);
       const float alpha = softmax_exp2(m - mnew);  // 0 on the first block (m = -inf)
@@ -238,8 +232,8 @@ __global__ __launch_bounds__(WAVES32 * kWave, 1) void attn_fwd_kernel(const floa
     psum = halves_sum(psum);
     l += psum;
     // O^T += V^T P^T ; step e uses key 8*(e/4) + 4h + e%4 = register e of s
-    const float* vrow0 = &Vt[buf][lq * VPITCH + 4 * lh];
-    const float* vrow1 = &Vt[buf][(32 + lq) * VPITCH + 4 * lh];
+    const float* vrow0 = Vt0 + buf * D * VPITCH + lq * VPITCH + 4 * lh;
+    const float* vrow1 = Vt0 + buf * D * VPITCH + (32 + lq) * VPITCH + 4 * lh;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const float4 a0 = *reinterpret_cast<const float4*>(vrow0 + 8 * j);
@@ -281,6 +275,315 @@ typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef short short4v __attribute__((ext_vector_type(4)));
 constexpr int KP16 = D + 8;        // K block pitch (halves): 144 B rows
 constexpr int VR16 = D + 8;        // V block pitch (halves), row-major: 144 B rows
+
+// fp32 storage on the fp16 matrix cores.  Every operand is scaled by a power of two and
+// split as x = hi + lo, hi = fp16(x), lo = fp16(x - hi) (22 significant bits), and each
+// product is accumulated in fp32 as hi.hi + hi.lo + lo.hi (Ootomo & Yokota, IJHPCA 2022,
+// restated for fp16 MFMA): three v_mfma_f32_32x32x16_f16 (32 cycles each) do what eight
+// v_mfma_f32_32x32x2f32 (64 cycles each) did.  The dropped lo.lo term and the rounding of lo
+// are below 2^-22 of the operands' size, the order of the fp32 sums' own rounding.
+//   Q  scaled per row (a lane owns a query), K and V by one power of two per head, taken
+//      from the head's first key block: its largest entry goes to [2^9, 2^10).  The
+//      logits' scale 2^-(..) is applied with the subtraction of the running maximum.
+//   P  formed as 2^(s - base) with base = running maximum - 7 (at most 2^15 at the lazy
+//      limit): 22 bits, or within 2^-32 of the largest probability for smaller ones.
+// A tile whose inputs the split does not represent to 22 bits (an entry past fp16's range
+// after scaling, 16 neighbouring entries of a row all below 2^-3 but not zero, a
+// non-finite entry, a scale out of range) is noticed while it is staged and computed
+// again by attend_tile_f32, so such inputs cost time, never accuracy.
+//   Layout: one 12-wave workgroup (384 queries, three waves per SIMD) per CU: the barrier
+// keeps the waves in step, where of three 4-wave workgroups on a CU the oldest finishes
+// first and the last runs alone.  Waves 0-7 stage: one float4 of K and one of V per
+// thread and 32-key block, loaded two blocks before they are split into LDS, which
+// happens while the logits' MFMAs run; a barrier every kGroup blocks.
+//   Bound by MFMA issue: B = 4, H = 16, T = 1370 (24 MFMAs, about 112 VALU instructions
+// per wave and block) 97 us = 317 TFLOP/s in fp32 terms; the fp32 MFMA tiles took 266 us
+// (116 TFLOP/s, 74 % of the fp32 peak).  Timing-only copies: 4 of the 24 MFMAs less
+// -12 %, no staging -8 %, no exponentials -6 %, no split of P -5 %, no maximum -1 %.
+// Measured and not kept: one block per barrier 102 us, four 97 us; the next block's
+// logits issued ahead of the softmax (164 VGPRs) 97 us, with the MFMAs and exponentials
+// interleaved by scheduling groups 100 us.  Error against float64: 4.3e-7 relative
+// (2-norm; 6.6e-7 for the fp32 MFMA tiles).
+constexpr int SP32 = D + 8;                    // pitch of a staged fp16 row: 144 bytes
+constexpr int kPlane = KB * SP32;              // halves of one plane; K hi, K lo, V hi, V lo
+constexpr int kGroup = 2;                      // key blocks between barriers: a ring of 2 kGroup slots
+constexpr int kSplitSmem = 2 * kGroup * 4 * kPlane * 2;
+constexpr int kF32KernelSmem = kSplitSmem > kF32Smem ? kSplitSmem : kF32Smem;
+constexpr float kPShift = 7.f;                 // probabilities are scaled by 2^7
+constexpr float kSplitMax = 60000.f;           // largest scaled entry (fp16 holds 65504)
+constexpr float kSplitMin = 0.125f;            // smallest scaled 16-entry group maximum: lo is exact to 2^-25
+
+// 2^k with x 2^k in [2^9, 2^10) for the largest |x| (given by its bits); 1 for zero or denormal
+__device__ inline float split_scale(uint32_t max_bits) {
+  const int e = (int)(max_bits >> 23);
+  return e == 0 ? 1.f : __uint_as_float((uint32_t)min(max(127 + 9 + 127 - e, 1), 254) << 23);
+}
+__device__ inline uint32_t abs_bits(float x) { return __float_as_uint(x) & 0x7fffffffu; }
+__device__ inline uint32_t abs_max4(const float (&x)[4]) {
+  return max(max(abs_bits(x[0]), abs_bits(x[1])), max(abs_bits(x[2]), abs_bits(x[3])));
+}
+// (a, b) -> hi = fp16 of each (one packed conversion, to nearest even), lo = fp16 of the exact
+// remainder x - hi (one mixed-precision fused multiply-add each, rounded once)
+typedef float float2v __attribute__((ext_vector_type(2)));
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+__device__ inline void split2(float a, float b, half2v& hi, half2v& lo) {
+  hi = __builtin_convertvector((float2v{a, b}), half2v);
+  asm("v_fma_mixlo_f16 %0, %1, -1.0, %2 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "=v"(lo) : "v"(hi), "v"(a));
+  asm("v_fma_mixhi_f16 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(lo) : "v"(hi), "v"(b));
+}
+
+__global__ __launch_bounds__(WAVES32 * kWave, 1) void attn_fwd_kernel(const float* __restrict__ qg,
+                                                                      const float* __restrict__ kg,
+                                                                      const float* __restrict__ vg,
+                                                                      float* __restrict__ og, int t, float scale_log2,
+                                                                      HeadLayout in, HeadLayout out, int nbh) {
+  __shared__ __attribute__((aligned(16))) unsigned char smem[kF32KernelSmem];
+  __shared__ uint32_t s_max[2][8];
+  _Float16* const planes = reinterpret_cast<_Float16*>(smem);
+
+  const int2 unit = fwd_unit<QW * WAVES32>(t, nbh);
+  if (unit.x < 0) return;
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  const int lq = lane & 31, lh = lane >> 5;
+  const int q = unit.y * (QW * WAVES32) + wave * QW + lq;
+  // waves whose 32 queries all lie past t only stage and synchronise
+  const bool active = unit.y * (QW * WAVES32) + wave * QW < t;
+  const long long head = in.base(unit.x), st = in.st;
+  const int nkb = (t + KB - 1) / KB;
+
+  // Staging: thread idx of waves 0-7 moves key idx/16, channels 4*(idx%16) of each block of
+  // K and of V through a buffer resource based at the block's first key whose extent ends
+  // with the last valid key (keys past t read zeros, offsets are loop-invariant).
+  static_assert(kGroup % 2 == 0, "block m's staging registers are set m % 2");
+  const bool stager = wave < 8;
+  const int idx = threadIdx.x & (KB * D / 4 - 1);
+  const int skey = idx / (D / 4), sd4 = 4 * (idx % (D / 4));
+  const uint32_t vo = (uint32_t)(((long long)skey * st + sd4) * 4);
+  auto load_block = [&](const float* src, int kb, float (&x)[4]) {
+    const long long rem = min(t - kb * KB, KB);  // valid keys of the block, >= 1
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(src + head + (long long)kb * KB * st), (short)0, (int)(((rem - 1) * st + D) * 4),
+        kBufferFlags);
+    const float4 v = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)vo, 0, 0));
+    x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w;
+  };
+  // staging registers, two sets: a block's loads are issued two steps before it is split
+  struct Staged {
+    float k[4], v[4];
+  };
+  Staged x0 = {}, x1 = {};
+  auto load_kv = [&](int kb, Staged& x) {  // past the last block: the last block again, never staged
+    load_block(kg, min(kb, nkb - 1), x.k);
+    load_block(vg, min(kb, nkb - 1), x.v);
+  };
+  if (stager) {
+    load_kv(0, x0);
+    load_kv(1, x1);
+  }
+  // this lane's query row: 8 m + lh halves of each 16-channel step, split, scaled by qscale
+  half8 qh[4], ql[4];
+  float qscale;
+  bool bad = false;  // this thread saw an entry the split does not represent
+  {
+    float qx[4][8];
+    uint32_t qmax = 0;
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        const float4 v = q < t ? *reinterpret_cast<const float4*>(qg + head + (long long)q * st + 16 * m + 8 * lh + 4 * g)
+                               : make_float4(0.f, 0.f, 0.f, 0.f);
+        qx[m][4 * g] = v.x; qx[m][4 * g + 1] = v.y; qx[m][4 * g + 2] = v.z; qx[m][4 * g + 3] = v.w;
+        const float q4[4] = {v.x, v.y, v.z, v.w};
+        qmax = max(qmax, abs_max4(q4));
+      }
+    {
+      const auto r = __builtin_amdgcn_permlane32_swap(qmax, qmax, false, false);
+      qmax = max(r[0], r[1]);
+    }
+    qscale = split_scale(qmax);
+    bad = qmax >= 0x7f800000u;
+    const float sgn = scale_log2 < 0.f ? -qscale : qscale;  // the logits' scale stays positive
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float v = qx[m][j] * sgn;
+        qh[m][j] = (_Float16)v;
+        ql[m][j] = (_Float16)(v - (float)qh[m][j]);
+      }
+  }
+  // the head's scales, from its first block
+  if (stager) {
+    uint32_t mk = abs_max4(x0.k), mv = abs_max4(x0.v);
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) {
+      mk = max(mk, (uint32_t)__shfl_xor((int)mk, off, kWave));
+      mv = max(mv, (uint32_t)__shfl_xor((int)mv, off, kWave));
+    }
+    if (lane == 0) {
+      s_max[0][wave] = mk;
+      s_max[1][wave] = mv;
+    }
+  }
+  __syncthreads();
+  uint32_t kmax = 0, vmax = 0;
+#pragma unroll
+  for (int w = 0; w < 8; ++w) {
+    kmax = max(kmax, s_max[0][w]);
+    vmax = max(vmax, s_max[1][w]);
+  }
+  const float kscale = split_scale(kmax), vscale = split_scale(vmax);
+  // c turns a product of scaled operands into log2 units; tiny scales (a zero softmax scale
+  // among them) are held at the smallest normal number, which moves no logit
+  const float c_raw = fabsf(scale_log2) / qscale / kscale;
+  bad = bad || !(c_raw < 0x1p100f);
+  const float c = fmaxf(c_raw, 0x1p-126f);
+
+  // splits this thread's K and V of a block into ring slot buf
+  auto stage = [&](int buf, const Staged& in_regs) {
+    _Float16* dst = planes + buf * 4 * kPlane + skey * SP32 + sd4;
+#pragma unroll
+    for (int op = 0; op < 2; ++op) {
+      float x[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[j] = op == 0 ? in_regs.k[j] * kscale : in_regs.v[j] * vscale;
+      // largest of 16 neighbouring entries of the row (four lanes); NaN and inf order last
+      int g = (int)abs_max4(x);
+      g = max(g, __builtin_amdgcn_update_dpp(0, g, 0xb1, 0xf, 0xf, false));
+      g = max(g, __builtin_amdgcn_update_dpp(0, g, 0x4e, 0xf, 0xf, false));
+      bad = bad || g > (int)__float_as_uint(kSplitMax) || (g < (int)__float_as_uint(kSplitMin) && g != 0);
+      half2v h0, h1, l0, l1;
+      split2(x[0], x[1], h0, l0);
+      split2(x[2], x[3], h1, l1);
+      *reinterpret_cast<half4*>(dst + 2 * op * kPlane) = half4{h0[0], h0[1], h1[0], h1[1]};
+      *reinterpret_cast<half4*>(dst + (2 * op + 1) * kPlane) = half4{l0[0], l0[1], l1[0], l1[1]};
+    }
+  };
+
+  floatx16 o0, o1;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    o0[v] = 0.f;
+    o1[v] = 0.f;
+  }
+  // base: running maximum of this lane's query minus kPShift; l: this half-wave's share of the sum
+  float base = -INFINITY, l = 0.f;
+  if (stager) {
+    for (int kb = 0; kb < kGroup && kb < nkb; kb += 2) {  // slots past the last block repeat it, unread
+      stage(kb, x0);
+      load_kv(kb + 2, x0);
+      stage(kb + 1, x1);
+      load_kv(kb + 3, x1);
+    }
+  }
+  // V^T fragments through the transposing read, as in the fp16 kernel below
+  const int vrd = (4 * lh + ((lq & 15) >> 2)) * SP32 + 16 * (lq >> 4) + 4 * (lq & 3);
+  auto step = [&](int kb, Staged& x) {
+    const _Float16* buf = planes + (kb & (2 * kGroup - 1)) * 4 * kPlane;
+    if ((kb & (kGroup - 1)) == 0) __syncthreads();
+    floatx16 s;
+    if (active) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) s[v] = 0.f;
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        const half8 kh = *reinterpret_cast<const half8*>(buf + lq * SP32 + 16 * m + 8 * lh);
+        const half8 kl = *reinterpret_cast<const half8*>(buf + kPlane + lq * SP32 + 16 * m + 8 * lh);
+        s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl, qh[m], s, 0, 0, 0);
+        s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, ql[m], s, 0, 0, 0);
+        s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh, qh[m], s, 0, 0, 0);
+      }
+    }
+    if (stager && kb + kGroup < nkb) {
+      // the other half of the ring was last read before this group's barrier
+      stage((kb + kGroup) & (2 * kGroup - 1), x);
+      load_kv(kb + kGroup + 2, x);
+    }
+    if (!active) return;
+    // register v holds key (v/4)*8 + 4h + v%4 of the block; only the last block is ragged
+    if ((kb + 1) * KB > t) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        if (kb * KB + (v >> 2) * 8 + lh * 4 + (v & 3) >= t) s[v] = -INFINITY;
+    }
+    float bmax = s[0];
+#pragma unroll
+    for (int v = 1; v < 16; ++v) bmax = __builtin_elementwise_maximum(bmax, s[v]);
+    bmax = halves_max(bmax) * c;
+    // lazy rescaling: the running maximum moves only past kLazyLog2
+    if (!__all(bmax <= base + (kPShift + kLazyLog2))) {
+      const float bnew = fmaxf(base, bmax - kPShift);
+      const float alpha = softmax_exp2(base - bnew);  // 0 on the first block (base = -inf)
+      l *= alpha;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        o0[v] *= alpha;
+        o1[v] *= alpha;
+      }
+      base = bnew;
+    }
+    half8 ph[2], pl[2];
+    float psum = 0.f;
+#pragma unroll
+    for (int v = 0; v < 16; v += 2) {
+      const float p0 = softmax_exp2(fmaf(s[v], c, -base)), p1 = softmax_exp2(fmaf(s[v + 1], c, -base));
+      psum += p0;
+      psum += p1;
+      half2v h, lo;
+      split2(p0, p1, h, lo);
+      ph[v >> 3][v & 7] = h[0];
+      ph[v >> 3][(v & 7) + 1] = h[1];
+      pl[v >> 3][v & 7] = lo[0];
+      pl[v >> 3][(v & 7) + 1] = lo[1];
+    }
+    l += psum;
+    typedef __attribute__((address_space(3))) short4v lds_short4v;
+    lds_short4v* const vb = (lds_short4v*)(buf + vrd);  // one address; the offsets below are immediates
+    auto tr = [&](int off) { return __builtin_bit_cast(half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(vb + off / 4)); };
+#pragma unroll
+    for (int mm = 0; mm < 2; ++mm) {
+      half8 vf[2][2];  // [plane][d half]
+#pragma unroll
+      for (int pn = 0; pn < 2; ++pn)
+#pragma unroll
+        for (int o = 0; o < 2; ++o) {
+          const int off = (2 + pn) * kPlane + 16 * mm * SP32 + 32 * o;
+          const half4 a = tr(off), b = tr(off + 8 * SP32);
+          vf[pn][o] = half8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+        }
+      o0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[1][0], ph[mm], o0, 0, 0, 0);
+      o1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[1][1], ph[mm], o1, 0, 0, 0);
+      o0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[0][0], pl[mm], o0, 0, 0, 0);
+      o1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[0][1], pl[mm], o1, 0, 0, 0);
+      o0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[0][0], ph[mm], o0, 0, 0, 0);
+      o1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[0][1], ph[mm], o1, 0, 0, 0);
+    }
+  };
+  for (int kb = 0; kb < nkb; kb += 2) {
+    step(kb, x0);
+    if (kb + 1 < nkb) step(kb + 1, x1);
+  }
+
+  // also the barrier before the buffers are reused
+  if (__syncthreads_or(bad)) {
+    attend_tile_f32(reinterpret_cast<float*>(smem), qg, kg, vg, og, t, scale_log2, in, out, unit);
+    return;
+  }
+  l = halves_sum(l);
+  if (q < t) {
+    const float inv = 1.f / l / vscale;
+    // register v of tile dt holds d = 32*dt + (v/4)*8 + 4h + v%4
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const float4 a = make_float4(o0[4 * g] * inv, o0[4 * g + 1] * inv, o0[4 * g + 2] * inv, o0[4 * g + 3] * inv);
+      const float4 b = make_float4(o1[4 * g] * inv, o1[4 * g + 1] * inv, o1[4 * g + 2] * inv, o1[4 * g + 3] * inv);
+      float* orow = og + out.base(unit.x) + (long long)q * out.st;
+      *reinterpret_cast<float4*>(orow + 8 * g + 4 * lh) = a;
+      *reinterpret_cast<float4*>(orow + 32 + 8 * g + 4 * lh) = b;
+    }
+  }
+}
 
 __global__ __launch_bounds__(WAVES * kWave) void attn_fwd_f16_kernel(const _Float16* __restrict__ qg,
                                                                      const _Float16* __restrict__ kg,
@@ -414,7 +717,6 @@ __global__ __launch_bounds__(WAVES * kWave) void attn_fwd_f16_kernel(const _Floa
   // block's probability sum enters l_run with its P V product.  Block j's K sits in
   // Ks[j & 1] from the top of step j - 2, its V in Vs[j & 1] from the top of step j;
   // every buffer is rewritten two barriers after its last read.
-  typedef _Float16 half2v __attribute__((ext_vector_type(2)));
   auto part_a = [&](int j, floatx16& s, float base, half8 (&pf_prev)[2], auto check_c) {
     if (decltype(check_c)::value && (j + 1) * KB > t) {  // only the last block is ragged
 #pragma unroll

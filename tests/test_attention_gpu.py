@@ -118,3 +118,70 @@ def test_config4_all_blocks(device, dtype):
         err = (out.double() - ref).abs().max().item()
         print(f'block {blk}: max |err| {err:.3e}', flush=True)
         assert err <= tol + tol * ref.abs().max().item(), (blk, err)
+
+
+def _f64(q, k, v, scale):
+    q, k, v = (x.detach().cpu().double() for x in (q, k, v))
+    return torch.softmax(torch.bmm(q * scale, k.transpose(1, 2).contiguous()), -1) @ v
+
+
+@pytest.mark.parametrize('t', [1, 31, 32, 33, 64, 65, 96, 129, 383, 384, 385, 417])
+def test_fp32_split_edges(device, t):
+    # key blocks, groups of blocks and 384-query tiles at their edges.  A logit is off by at most a
+    # few 2^-22 |q||k| scale (about 5e-6 here at |q| |k| = 26 and scale 1/8), and the output by that
+    # times the spread of v; fp32 sums of 417 terms add less
+    g = torch.Generator().manual_seed(t)
+    q, k, v = (torch.randn((3, t, 64), generator=g) * 0.64 for _ in range(3))
+    out = _attention_hip.attention(q.to(device), k.to(device), v.to(device), 0.125).cpu().double()
+    torch.testing.assert_close(out, _f64(q, k, v, 0.125), rtol=0, atol=1e-5)
+
+
+@pytest.mark.parametrize('change', ['v_rows', 'k_rows', 'tiny_v', 'huge_k', 'first_block_zero', 'q_rows', 'none'])
+@pytest.mark.parametrize('scale', [0.125, -0.125, 0.0])
+def test_fp32_inputs_outside_the_split_range(device, change, scale):
+    # rows far larger or smaller than the head's first block, which the fp16 split does not hold to
+    # 22 bits: those tiles are computed in fp32, so the result stays an fp32 result everywhere
+    g = torch.Generator().manual_seed(len(change))
+    q, k, v = (torch.randn((2, 200, 64), generator=g) for _ in range(3))
+    if change == 'v_rows':
+        v[0, 100:] *= 1e6
+        v[1, 40] *= 1e-7
+    elif change == 'k_rows':
+        k[0, 70] *= 1e-6
+        k[1, 150:160] *= 30.0
+    elif change == 'tiny_v':
+        v *= 1e-30
+    elif change == 'huge_k':
+        k, q = k * 1e25, q * 1e-25
+    elif change == 'first_block_zero':
+        k[:, :32] = 0
+        v[:, :32] = 0
+        k[1, 32:] *= 1e-4
+        v[1, 32:] *= 1e-4
+    elif change == 'q_rows':
+        q[:, ::7] *= 1e-12
+    out = _attention_hip.attention(q.to(device), k.to(device), v.to(device), scale).cpu().double()
+    ref = _f64(q, k, v, scale)
+    # relative to the largest value each output is a mean of: logits within 2^-20 of |q||k| scale
+    span = (q.double().norm(dim=-1).max() * k.double().norm(dim=-1).max()).item() * abs(scale)
+    tol = (2.0 ** -20 * max(span, 1.0)) * v.abs().amax((1, 2), keepdim=True).double()
+    assert torch.all((out - ref).abs() <= tol), ((out - ref).abs() / tol).max()
+
+
+@pytest.mark.parametrize('where', ['q', 'k', 'v'])
+@pytest.mark.parametrize('value', [float('nan'), float('inf'), -float('inf')])
+def test_fp32_non_finite_entries(device, where, value):
+    # a non-finite entry of one head: that head as fp32 arithmetic gives it (NaN and infinities where
+    # torch's fp32 softmax has them), the other head untouched
+    g = torch.Generator().manual_seed(5)
+    q, k, v = (torch.randn((2, 77, 64), generator=g) for _ in range(3))
+    {'q': q, 'k': k, 'v': v}[where][1, 50, 3] = value
+    out = _attention_hip.attention(q.to(device), k.to(device), v.to(device), 0.125).cpu()
+    ref = reference(q, k, v, 0.125)
+    torch.testing.assert_close(out[0], ref[0], rtol=1e-4, atol=2e-5)
+    if where != 'k':      # a +-inf key gives some queries a -inf logit, whose NaN the two maxima treat alike
+        torch.testing.assert_close(out[1], ref[1], rtol=1e-4, atol=2e-5, equal_nan=True)
+    else:
+        sure = ~torch.isfinite(ref[1])
+        assert not torch.isfinite(out[1][sure]).any()
+        torch.testing.assert_close(out[1][~sure], ref[1][~sure], rtol=1e-4, atol=2e-5)
