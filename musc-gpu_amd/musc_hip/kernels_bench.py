@@ -249,7 +249,8 @@ def bench_attention(args):
     ms_host = sum(ts_host) / len(ts_host)
     flop = 4.0 * B * H * T * T * D
     tf = flop / (ms / 1e3) / 1e12
-    peak = FP32_MFMA_TFLOPS if dtype == torch.float32 else FP16_MFMA_TFLOPS
+    # fp32 storage runs three fp16 MFMA products per product
+    peak = FP16_MFMA_TFLOPS / 3 if dtype == torch.float32 else FP16_MFMA_TFLOPS
     return {'kernel': 'attention', 'dtype': args.dtype, 'B': B, 'H': H, 'T': T, 'D': D, 'blocks': args.blocks,
             'avg_ms_per_block': ms, 'flop_per_block': flop, 'tflops': tf, 'frac_mfma_peak': tf / peak,
             'peak_tflops': peak, 'host_paced_ms_per_block': ms_host,
