@@ -118,7 +118,8 @@ int musc_msm_nearest_f32(const float* z, int n, int p, int c, float* nearest,
 /* The four stages of musc_msm_scores_f32, for callers that time or overlap
  * them separately (same arguments and workspace):
  *   prepare      row norms ||z||^2 (and, with MUSC_MSM_NORMALIZE_ROWS, the row
- *                scales 1/||z||) and the +inf fill of the minima buffer;
+ *                scales 1/||z||) and the +inf fill of the minima buffer, and each
+ *                image's largest norm;
  *   pair_minima  fp32-MFMA pairwise distances of every unordered patch pair of
  *                different images, reduced along rows and columns into the
  *                per-(patch, image) minima (the hot kernel);
@@ -164,6 +165,21 @@ int musc_msm_split_pair_minima(int n, int p, int c, void* workspace, size_t work
                                hipStream_t stream);
 int musc_msm_split_scores_f32(const float* z, int n, int p, int c, int rank_lo, int rank_hi,
                               int flags, double* scores, void* workspace,
+                              size_t workspace_bytes, hipStream_t stream);
+
+/* Mutual scores of `pools` pools of one shape, one launch per stage over all of them:
+ * what a division scores, every (radius, layer) pool of its LNAMD features.
+ *   z       (pools, n, p, c) fp32, scores (pools, n, p) float64, both contiguous; each
+ *           pool's scores are those of musc_msm_scores_f32 (MUSC_MSM_ENGINE_F32) or
+ *           musc_msm_split_scores_f32 (MUSC_MSM_ENGINE_SPLIT16) with the same flags.
+ *   workspace   musc_msm_pools_workspace_bytes: one pool's workspace per pool.  A caller
+ *           bounds it by scoring a few pools at a time.
+ * The reference scores the layers and radii one after another (models/musc.py:227-256). */
+#define MUSC_MSM_ENGINE_F32 0
+#define MUSC_MSM_ENGINE_SPLIT16 1
+int musc_msm_pools_workspace_bytes(int pools, int n, int p, int c, int engine, size_t* out);
+int musc_msm_pools_scores_f32(const float* z, int pools, int n, int p, int c, int rank_lo, int rank_hi,
+                              int flags, int engine, double* scores, void* workspace,
                               size_t workspace_bytes, hipStream_t stream);
 
 /* ------------------------------------------------------------------------ */

@@ -5,8 +5,9 @@
 // score is the mean of ascending ranks [a, b) of {d(q, j)}_{j != i}.
 //
 // MI355X design
-//   1. msm_norms_kernel      ||z_row||^2 for all n*p rows (one wave per row).
-//   2. fill                  per-(row, image) minima buffer := +inf bits.
+//   1. msm_norms_kernel      ||z_row||^2 for all n*p rows (one wave per row), and the row's
+//                            keys of the per-(row, image) minima buffer := +inf.
+//   2. image_max_kernel      each image's largest norm (for the refinement).
 //   3. msm_pair_min_kernel   (msm_pair.hip) the whole pool is one (n*p) x (n*p) Gram
 //                            matrix; the upper triangle of 128x128 tiles on fp32
 //                            MFMA, each tile reduced along rows and columns into
@@ -18,6 +19,11 @@
 //                            merged by a bitonic network), or the a-th and b-th
 //                            smallest by a binary search over the key bits (one
 //                            lane per patch for n <= 192, one wave per patch beyond).
+// Every kernel takes several pools of one shape in gridDim.y: the pools of a division's
+// layers and radii go through one launch per stage, because a few small images leave most
+// of the chip idle in each launch (45 workgroups of the pair kernel for one pool of eight
+// 12 x 12 images): tokens to maps of eight such images, two layers and two radii, 168.6 us
+// pool by pool (29 launches), 65.3 us together (10).
 #include <mutex>
 
 #include "msm_common.hpp"
@@ -32,13 +38,13 @@ namespace msm {
 // treated as z / ||z|| (the L2 normalisation of models/musc.py:238 applied on the
 // fly): inv[row] = 1 / ||z_row|| and norms[row] = ||z_row||^2 * inv^2.  scale[row]
 // (the refinement's row scale) = inv[row].
-__global__ __launch_bounds__(256) void msm_norms_kernel(const float* __restrict__ z, int rows, int c,
-                                                        int normalize, float* __restrict__ norms,
-                                                        float* __restrict__ inv, float* __restrict__ scale) {
+__global__ __launch_bounds__(256) void msm_norms_kernel(const float* __restrict__ z, int rows, int n, int c,
+                                                        int normalize, Workspace w, size_t ws_step) {
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
   const long long row = (long long)blockIdx.x * (blockDim.x / kWave) + wave;
   if (row >= rows) return;
-  const double acc = row_sumsq(z + row * (long long)c, c, lane);
+  fill_row_keys(pool_ptr(w.minbits, ws_step) + row * n, n, lane);
+  const double acc = row_sumsq(z + (blockIdx.y * (long long)rows + row) * c, c, lane);
   if (lane == 0) {
     float nrm, s;
     if (normalize) {
@@ -49,9 +55,9 @@ __global__ __launch_bounds__(256) void msm_norms_kernel(const float* __restrict_
       s = 1.f;
       nrm = (float)acc;
     }
-    inv[row] = s;
-    scale[row] = s;
-    norms[row] = nrm;
+    pool_ptr(w.inv, ws_step)[row] = s;
+    pool_ptr(w.scale, ws_step)[row] = s;
+    pool_ptr(w.norms, ws_step)[row] = nrm;
   }
 }
 
@@ -79,7 +85,9 @@ constexpr int kRankChunk = 32;
 template <int kKeys>
 __global__ __launch_bounds__(kRankRows) void msm_rank_select_kernel(const uint32_t* __restrict__ minbits, int rows,
                                                                     int n, int p, int a, int b,
-                                                                    double* __restrict__ scores) {
+                                                                    double* __restrict__ scores, size_t ws_step) {
+  minbits = pool_ptr(minbits, ws_step);
+  scores += blockIdx.y * (long long)rows;
   __shared__ uint32_t s_chunk[kRankRows * (kRankChunk + 1)];
   const int t = threadIdx.x;
   const long long row0 = (long long)blockIdx.x * kRankRows;
@@ -173,7 +181,9 @@ constexpr int kRank2Rows = 32;
 template <int kList>
 __global__ __launch_bounds__(kWave) void msm_rank_insert2_kernel(const uint32_t* __restrict__ minbits, int rows,
                                                                  int n, int p, int a, int b,
-                                                                 double* __restrict__ scores) {
+                                                                 double* __restrict__ scores, size_t ws_step) {
+  minbits = pool_ptr(minbits, ws_step);
+  scores += blockIdx.y * (long long)rows;
   constexpr int N2 = kList <= 8 ? 8 : (kList <= 16 ? 16 : 32);
   extern __shared__ __attribute__((aligned(16))) uint32_t s_rowkeys[];  // kRank2Rows * n
   const int t = threadIdx.x;
@@ -251,7 +261,10 @@ constexpr int kMaxSelectKeys = 192;
 
 template <int kSlots>
 __global__ __launch_bounds__(kRankWaves * kWave) void msm_rank_wave_kernel(
-    const uint32_t* __restrict__ minbits, int rows, int n, int p, int a, int b, double* __restrict__ scores) {
+    const uint32_t* __restrict__ minbits, int rows, int n, int p, int a, int b, double* __restrict__ scores,
+    size_t ws_step) {
+  minbits = pool_ptr(minbits, ws_step);
+  scores += blockIdx.y * (long long)rows;
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
   const long long row = (long long)blockIdx.x * kRankWaves + wave;
   if (row >= rows) return;
@@ -391,7 +404,12 @@ __global__ __launch_bounds__(256) void msm_refine_kernel(const float* __restrict
                                                          const float* __restrict__ norms,
                                                          const float* __restrict__ scale,
                                                          const uint32_t* __restrict__ imgmax,
-                                                         uint32_t* __restrict__ minbits, float thr) {
+                                                         uint32_t* __restrict__ minbits, float thr, size_t ws_step) {
+  z += blockIdx.y * (long long)rows * c;
+  norms = pool_ptr(norms, ws_step);
+  scale = pool_ptr(scale, ws_step);
+  imgmax = pool_ptr(imgmax, ws_step);
+  minbits = pool_ptr(minbits, ws_step);
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
   const long long row0 = ((long long)blockIdx.x * (blockDim.x / kWave) + wave) * kRefineRows;
   if (row0 >= rows) return;
@@ -436,32 +454,34 @@ inline int validate(const float* z, int n, int p, int c, void* ws, size_t ws_byt
   return MUSC_OK;
 }
 
-// Stage 1: row norms and the +inf fill of the minima buffer.
-inline void run_prepare(const float* z, int n, int p, int c, int normalize, const Workspace& w, hipStream_t s) {
+// Stage 1: row norms, scales and the +inf fill of the minima buffer, then the image maxima.
+void run_prepare(const float* z, int n, int p, int c, int normalize, const Workspace& w, const Pools& pools,
+                 hipStream_t s) {
   const long long rows = (long long)n * p;
-  hipLaunchKernelGGL(msm_norms_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, z, (int)rows, c,
-                     normalize, w.norms, w.inv, w.scale);
-  launch_image_max(w.norms, n, p, w.imgmax, s);
-  launch_fill_u32(w.minbits, (size_t)rows * n, kMinFill, s);
+  hipLaunchKernelGGL(msm_norms_kernel, dim3((unsigned)((rows + 3) / 4), pools.count), dim3(256), 0, s, z, (int)rows, n,
+                     c, normalize, w, pools.ws_step);
+  launch_image_max(w.norms, n, p, w.imgmax, pools, s);
 }
 
 // Stage 3: exact minima where the expanded form cancels (either engine's keys).
-int run_refine(const float* z, int n, int p, int c, const Workspace& w, hipStream_t s) {
+int run_refine(const float* z, int n, int p, int c, const Workspace& w, const Pools& pools, hipStream_t s) {
   const long long rows = (long long)n * p;
   const long long blocks = ((rows + kRefineRows - 1) / kRefineRows + 3) / 4;
-  hipLaunchKernelGGL(msm_refine_kernel, dim3((unsigned)blocks), dim3(256), 0, s, z, (int)rows, n, p, c, w.norms,
-                     w.scale, w.imgmax, w.minbits, fmaxf(32.f * (float)c, kRefineFloor) * kRefineEps);
+  hipLaunchKernelGGL(msm_refine_kernel, dim3((unsigned)blocks, pools.count), dim3(256), 0, s, z, (int)rows, n, p, c,
+                     w.norms, w.scale, w.imgmax, w.minbits, fmaxf(32.f * (float)c, kRefineFloor) * kRefineEps,
+                     pools.ws_step);
   return check_launch();
 }
 
 // Stage 4: trimmed rank means.
-int run_rank(int n, int p, int a, int b, double* scores, const Workspace& w, hipStream_t s) {
+int run_rank(int n, int p, int a, int b, double* scores, const Workspace& w, const Pools& pools, hipStream_t s) {
   const long long rows = (long long)n * p;
   if (n <= kMaxSelectKeys && b <= 32) {
-    const dim3 grid((unsigned)((rows + kRank2Rows - 1) / kRank2Rows)), block(kWave);
+    const dim3 grid((unsigned)((rows + kRank2Rows - 1) / kRank2Rows), pools.count), block(kWave);
     const size_t smem = (size_t)kRank2Rows * n * sizeof(uint32_t);  // <= 24 KB
 #define MUSC_RANK_INSERT(K) \
-  hipLaunchKernelGGL(msm_rank_insert2_kernel<K>, grid, block, smem, s, w.minbits, (int)rows, n, p, a, b, scores)
+  hipLaunchKernelGGL(msm_rank_insert2_kernel<K>, grid, block, smem, s, w.minbits, (int)rows, n, p, a, b, scores, \
+                     pools.ws_step)
     if (b <= 8) MUSC_RANK_INSERT(8);
     else if (b <= 16) MUSC_RANK_INSERT(16);
     else if (b <= 24) MUSC_RANK_INSERT(24);
@@ -470,10 +490,11 @@ int run_rank(int n, int p, int a, int b, double* scores, const Workspace& w, hip
     return check_launch();
   }
   if (n <= kMaxSelectKeys) {
-    const dim3 grid((unsigned)((rows + kRankRows - 1) / kRankRows)), block(kRankRows);
+    const dim3 grid((unsigned)((rows + kRankRows - 1) / kRankRows), pools.count), block(kRankRows);
     const size_t smem = 0;  // the chunk buffer is static
 #define MUSC_RANK_LAUNCH(K) \
-  hipLaunchKernelGGL(msm_rank_select_kernel<K>, grid, block, smem, s, w.minbits, (int)rows, n, p, a, b, scores)
+  hipLaunchKernelGGL(msm_rank_select_kernel<K>, grid, block, smem, s, w.minbits, (int)rows, n, p, a, b, scores, \
+                     pools.ws_step)
     if (n <= 32) MUSC_RANK_LAUNCH(32);
     else if (n <= 64) MUSC_RANK_LAUNCH(64);
     else if (n <= 96) MUSC_RANK_LAUNCH(96);
@@ -483,9 +504,10 @@ int run_rank(int n, int p, int a, int b, double* scores, const Workspace& w, hip
 #undef MUSC_RANK_LAUNCH
     return check_launch();
   }
-  const dim3 grid((unsigned)((rows + kRankWaves - 1) / kRankWaves)), block(kRankWaves * kWave);
+  const dim3 grid((unsigned)((rows + kRankWaves - 1) / kRankWaves), pools.count), block(kRankWaves * kWave);
 #define MUSC_RANK_WAVE(K) \
-  hipLaunchKernelGGL(msm_rank_wave_kernel<K>, grid, block, 0, s, w.minbits, (int)rows, n, p, a, b, scores)
+  hipLaunchKernelGGL(msm_rank_wave_kernel<K>, grid, block, 0, s, w.minbits, (int)rows, n, p, a, b, scores, \
+                     pools.ws_step)
   if (n <= 256) MUSC_RANK_WAVE(4);
   else if (n <= 512) MUSC_RANK_WAVE(8);
   else if (n <= 1024) MUSC_RANK_WAVE(16);
@@ -511,7 +533,8 @@ extern "C" int musc_msm_prepare_f32(const float* z, int n, int p, int c, int fla
   int rc = msm::validate(z, n, p, c, workspace, workspace_bytes);
   if (rc) return rc;
   if (flags & ~MUSC_MSM_NORMALIZE_ROWS) return MUSC_ERR_INVALID_ARG;
-  msm::run_prepare(z, n, p, c, (flags & MUSC_MSM_NORMALIZE_ROWS) ? 1 : 0, msm::carve(workspace, n, p), stream);
+  msm::run_prepare(z, n, p, c, (flags & MUSC_MSM_NORMALIZE_ROWS) ? 1 : 0, msm::carve(workspace, n, p), msm::kOnePool,
+                   stream);
   return check_launch();
 }
 
@@ -519,14 +542,14 @@ extern "C" int musc_msm_pair_minima_f32(const float* z, int n, int p, int c, voi
                                         size_t workspace_bytes, hipStream_t stream) {
   int rc = msm::validate(z, n, p, c, workspace, workspace_bytes);
   if (rc) return rc;
-  return msm::run_pairs(z, n, p, c, msm::carve(workspace, n, p), stream);
+  return msm::run_pairs(z, n, p, c, msm::carve(workspace, n, p), msm::kOnePool, stream);
 }
 
 extern "C" int musc_msm_refine_f32(const float* z, int n, int p, int c, void* workspace, size_t workspace_bytes,
                                    hipStream_t stream) {
   int rc = msm::validate(z, n, p, c, workspace, workspace_bytes);
   if (rc) return rc;
-  return msm::run_refine(z, n, p, c, msm::carve(workspace, n, p), stream);
+  return msm::run_refine(z, n, p, c, msm::carve(workspace, n, p), msm::kOnePool, stream);
 }
 
 extern "C" int musc_msm_rank_f32(int n, int p, int rank_lo, int rank_hi, double* scores, void* workspace,
@@ -535,7 +558,7 @@ extern "C" int musc_msm_rank_f32(int n, int p, int rank_lo, int rank_hi, double*
   if (n > 4096 || (long long)n * p > (1LL << 30)) return MUSC_ERR_UNSUPPORTED;
   if (!workspace || workspace_bytes < msm::workspace_bytes(n, p)) return MUSC_ERR_WORKSPACE;
   if (!msm::ws_aligned(workspace)) return MUSC_ERR_INVALID_ARG;
-  return msm::run_rank(n, p, rank_lo, rank_hi, scores, msm::carve(workspace, n, p), stream);
+  return msm::run_rank(n, p, rank_lo, rank_hi, scores, msm::carve(workspace, n, p), msm::kOnePool, stream);
 }
 
 extern "C" int musc_msm_scores_f32(const float* z, int n, int p, int c, int rank_lo, int rank_hi,
@@ -545,12 +568,59 @@ extern "C" int musc_msm_scores_f32(const float* z, int n, int p, int c, int rank
   if (rc) return rc;
   if (!scores || rank_lo < 0 || rank_lo >= rank_hi || rank_hi > n - 1) return MUSC_ERR_INVALID_ARG;
   const msm::Workspace w = msm::carve(workspace, n, p);
-  msm::run_prepare(z, n, p, c, 0, w, stream);
-  rc = msm::run_pairs(z, n, p, c, w, stream);
+  msm::run_prepare(z, n, p, c, 0, w, msm::kOnePool, stream);
+  rc = msm::run_pairs(z, n, p, c, w, msm::kOnePool, stream);
   if (rc) return rc;
-  rc = msm::run_refine(z, n, p, c, w, stream);
+  rc = msm::run_refine(z, n, p, c, w, msm::kOnePool, stream);
   if (rc) return rc;
-  return msm::run_rank(n, p, rank_lo, rank_hi, scores, w, stream);
+  return msm::run_rank(n, p, rank_lo, rank_hi, scores, w, msm::kOnePool, stream);
+}
+
+// ---------------------------------------------------------------------------
+// Several pools of one shape: one launch per stage over all of them.
+// ---------------------------------------------------------------------------
+namespace {
+
+size_t pool_step(int n, int p, int c, int engine) {
+  return engine == MUSC_MSM_ENGINE_SPLIT16 ? msm::split::pool_workspace_bytes(n, p, c) : msm::workspace_bytes(n, p);
+}
+
+}  // namespace
+
+extern "C" int musc_msm_pools_workspace_bytes(int pools, int n, int p, int c, int engine, size_t* out) {
+  if (!out || pools < 1 || n < 2 || p < 1 || c < 1) return MUSC_ERR_INVALID_ARG;
+  if (engine != MUSC_MSM_ENGINE_F32 && engine != MUSC_MSM_ENGINE_SPLIT16) return MUSC_ERR_INVALID_ARG;
+  *out = (size_t)pools * pool_step(n, p, c, engine);
+  return MUSC_OK;
+}
+
+extern "C" int musc_msm_pools_scores_f32(const float* z, int pools, int n, int p, int c, int rank_lo, int rank_hi,
+                                         int flags, int engine, double* scores, void* workspace,
+                                         size_t workspace_bytes, hipStream_t stream) {
+  if (pools < 1 || (engine != MUSC_MSM_ENGINE_F32 && engine != MUSC_MSM_ENGINE_SPLIT16)) return MUSC_ERR_INVALID_ARG;
+  if (flags & ~MUSC_MSM_NORMALIZE_ROWS) return MUSC_ERR_INVALID_ARG;
+  int rc = msm::validate(z, n, p, c, workspace, workspace_bytes);
+  if (rc) return rc;
+  if (pools > 65535) return MUSC_ERR_UNSUPPORTED;  // gridDim.y
+  if (workspace_bytes < (size_t)pools * pool_step(n, p, c, engine)) return MUSC_ERR_WORKSPACE;
+  if (!scores || rank_lo < 0 || rank_lo >= rank_hi || rank_hi > n - 1) return MUSC_ERR_INVALID_ARG;
+  if (engine == MUSC_MSM_ENGINE_SPLIT16 && p < 256) return MUSC_ERR_UNSUPPORTED;
+  const msm::Pools many{pools, pool_step(n, p, c, engine)};
+  const msm::Workspace w = msm::carve(workspace, n, p);
+  const int normalize = (flags & MUSC_MSM_NORMALIZE_ROWS) ? 1 : 0;
+  if (engine == MUSC_MSM_ENGINE_SPLIT16) {
+    rc = msm::split::validate(n, p, c, workspace, workspace_bytes);
+    if (rc) return rc;
+    msm::split::run_prepare(z, n, p, c, normalize, workspace, many, stream);
+    rc = msm::split::run_pairs(n, p, c, workspace, many, stream);
+  } else {
+    msm::run_prepare(z, n, p, c, normalize, w, many, stream);
+    rc = msm::run_pairs(z, n, p, c, w, many, stream);
+  }
+  if (rc) return rc;
+  rc = msm::run_refine(z, n, p, c, w, many, stream);
+  if (rc) return rc;
+  return msm::run_rank(n, p, rank_lo, rank_hi, scores, w, many, stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -607,10 +677,10 @@ extern "C" int musc_msm_nearest_f32(const float* z, int n, int p, int c, float* 
   if (rc) return rc;
   if (!nearest) return MUSC_ERR_INVALID_ARG;
   const msm::Workspace w = msm::carve(workspace, n, p);
-  msm::run_prepare(z, n, p, c, 0, w, stream);
-  rc = msm::run_pairs(z, n, p, c, w, stream);
+  msm::run_prepare(z, n, p, c, 0, w, msm::kOnePool, stream);
+  rc = msm::run_pairs(z, n, p, c, w, msm::kOnePool, stream);
   if (rc) return rc;
-  rc = msm::run_refine(z, n, p, c, w, stream);
+  rc = msm::run_refine(z, n, p, c, w, msm::kOnePool, stream);
   if (rc) return rc;
   const size_t count = (size_t)n * p * n;
   const size_t blocks = (count + 255) / 256 < 65536 ? (count + 255) / 256 : 65536;  // grid-stride beyond

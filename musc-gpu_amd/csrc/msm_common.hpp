@@ -82,6 +82,11 @@ __device__ inline int2 decode_tile(long long w, long long T) {
   return make_int2((int)(I0 + q % h), (int)(I0 + h + q / h));
 }
 
+// +inf keys for one row of the minima buffer, by the wave that owns the row.
+__device__ inline void fill_row_keys(uint32_t* __restrict__ keys, int n, int lane) {
+  for (int j = lane; j < n; j += kWave) keys[j] = kMinFill;
+}
+
 // Sum of squares of one row in fp64, reduced over the wave (result in every lane).
 __device__ inline double row_sumsq(const float* __restrict__ src, int c, int lane) {
   double acc = 0.0;
@@ -177,6 +182,22 @@ inline size_t workspace_bytes(long long n, long long p) {
   return 3 * align_up((size_t)rows * 4, 256) + align_up((size_t)rows * n * 4, 256) + align_up((size_t)n * 4, 256);
 }
 
+// A launch over several pools of one shape: gridDim.y pools, pool k's features z + k * z_step
+// and workspace `ws_step` bytes after pool k - 1's (both 0 for one pool).
+struct Pools {
+  int count;
+  size_t ws_step;
+};
+constexpr Pools kOnePool{1, 0};
+
+// (byte-pointer arithmetic: through an integer the compiler forgets that the memory is
+// global and issues flat accesses)
+template <typename T>
+__device__ inline T* pool_ptr(T* base, size_t ws_step) {
+  typedef typename std::conditional<std::is_const<T>::value, const char, char>::type byte;
+  return reinterpret_cast<T*>(reinterpret_cast<byte*>(base) + blockIdx.y * ws_step);
+}
+
 inline Workspace carve(void* ws, long long n, long long p) {
   const long long rows = n * p;
   const size_t vec = align_up((size_t)rows * 4, 256);
@@ -195,9 +216,9 @@ inline Workspace carve(void* ws, long long n, long long p) {
 // pairs): one workgroup per image, no atomics.
 template <int kUnused = 0>
 __global__ __launch_bounds__(256) void image_max_kernel(const float* __restrict__ norms, int p,
-                                                        uint32_t* __restrict__ imgmax) {
+                                                        uint32_t* __restrict__ imgmax, size_t ws_step) {
   __shared__ float part[256 / kWave];
-  const float* src = norms + (long long)blockIdx.x * p;
+  const float* src = pool_ptr(norms, ws_step) + (long long)blockIdx.x * p;
   float m = 0.f;
   for (int q = threadIdx.x; q < p; q += 256) {
     const float v = src[q];
@@ -208,23 +229,36 @@ __global__ __launch_bounds__(256) void image_max_kernel(const float* __restrict_
   __syncthreads();
   if (threadIdx.x == 0) {
     for (int w = 1; w < 256 / kWave; ++w) m = fmaxf(m, part[w]);
-    imgmax[blockIdx.x] = __float_as_uint(m);
+    pool_ptr(imgmax, ws_step)[blockIdx.x] = __float_as_uint(m);
   }
 }
 
-inline void launch_image_max(const float* norms, int n, int p, uint32_t* imgmax, hipStream_t s) {
-  hipLaunchKernelGGL(image_max_kernel<0>, dim3((unsigned)n), dim3(256), 0, s, norms, p, imgmax);
+inline void launch_image_max(const float* norms, int n, int p, uint32_t* imgmax, const Pools& pools, hipStream_t s) {
+  hipLaunchKernelGGL(image_max_kernel<0>, dim3((unsigned)n, pools.count), dim3(256), 0, s, norms, p, imgmax,
+                     pools.ws_step);
 }
 
 // The fp32 MFMA pair-minima kernel (msm_pair.hip): leaves the squared minima keys.
-int run_pairs(const float* z, int n, int p, int c, const Workspace& w, hipStream_t s);
+int run_pairs(const float* z, int n, int p, int c, const Workspace& w, const Pools& pools, hipStream_t s);
 
 // Trimmed rank means over the minima (defined in msm.hip, shared by both engines).
-int run_rank(int n, int p, int a, int b, double* scores, const Workspace& w, hipStream_t s);
+int run_rank(int n, int p, int a, int b, double* scores, const Workspace& w, const Pools& pools, hipStream_t s);
 
 // Exact distances for the minima the expanded form cannot resolve (defined in
 // msm.hip, shared by both engines; runs after either pair kernel).
-int run_refine(const float* z, int n, int p, int c, const Workspace& w, hipStream_t s);
+int run_refine(const float* z, int n, int p, int c, const Workspace& w, const Pools& pools, hipStream_t s);
+
+// Row norms, scales, image maxima and the +inf fill of the minima keys (defined in msm.hip).
+void run_prepare(const float* z, int n, int p, int c, int normalize, const Workspace& w, const Pools& pools,
+                 hipStream_t s);
+
+// The split engine's stages over several pools (msm_split.hip).
+namespace split {
+size_t pool_workspace_bytes(long long n, long long p, int c);
+int validate(int n, int p, int c, void* ws, size_t ws_bytes);
+void run_prepare(const float* z, int n, int p, int c, int normalize, void* ws, const Pools& pools, hipStream_t s);
+int run_pairs(int n, int p, int c, void* ws, const Pools& pools, hipStream_t s);
+}  // namespace split
 
 }  // namespace msm
 }  // namespace musc

@@ -93,7 +93,7 @@ __device__ inline void store_chunk(float* __restrict__ dst, const stage4 (&reg)[
 template <int kLoad, bool kSplit>
 __global__ __launch_bounds__(THREADS, kSplit ? 3 : 2) void msm_pair_min_kernel(
     const float* __restrict__ z, const float* __restrict__ norms, const float* __restrict__ inv,
-    uint32_t* __restrict__ minbits, int rows, int n, int p, int c, int T, long long ntiles) {
+    uint32_t* __restrict__ minbits, int rows, int n, int p, int c, int T, long long ntiles, size_t ws_step) {
   __shared__ __attribute__((aligned(16))) float smem[kSplit ? kStageFloats : kSmemFloats];
   __shared__ __attribute__((aligned(16))) float s_rnorm[BM];
   __shared__ __attribute__((aligned(16))) float s_cnorm[BN];
@@ -112,6 +112,10 @@ __global__ __launch_bounds__(THREADS, kSplit ? 3 : 2) void msm_pair_min_kernel(
   const int rimg0 = row0 / p, cimg0 = col0 / p;
   const bool simple = (row0 + BM <= rows) && (col0 + BN <= rows) && (rlast / p == rimg0) && (clast / p == cimg0);
   if (simple && rimg0 == cimg0) return;
+  z += blockIdx.y * (long long)rows * c;  // this workgroup's pool
+  norms = pool_ptr(norms, ws_step);
+  inv = pool_ptr(inv, ws_step);
+  minbits = pool_ptr(minbits, ws_step);
 
   const int t = threadIdx.x;
   if (t < BM) {
@@ -507,15 +511,15 @@ __global__ __launch_bounds__(THREADS, kSplit ? 3 : 2) void msm_pair_min_kernel(
 }
 
 // Stage 2: the fp32 MFMA pairwise-minima kernel (leaves squared minima bits).
-int run_pairs(const float* z, int n, int p, int c, const Workspace& w, hipStream_t s) {
+int run_pairs(const float* z, int n, int p, int c, const Workspace& w, const Pools& pools, hipStream_t s) {
   const long long rows = (long long)n * p;
   const long long T = (rows + BM - 1) / BM;
   const long long ntiles = total_tiles(T);
   const long long grid = (ntiles + kXcds - 1) / kXcds * kXcds;
   if (grid > 0x7fffffffLL) return MUSC_ERR_UNSUPPORTED;
 #define MUSC_PAIR_LAUNCH(V4, SPLIT)                                                                              \
-  hipLaunchKernelGGL((msm_pair_min_kernel<V4, SPLIT>), dim3((unsigned)grid), dim3(THREADS), 0, s, z, w.norms, w.inv, \
-                     w.minbits, (int)rows, n, p, c, (int)T, ntiles)
+  hipLaunchKernelGGL((msm_pair_min_kernel<V4, SPLIT>), dim3((unsigned)grid, pools.count), dim3(THREADS), 0, s, z,    \
+                     w.norms, w.inv, w.minbits, (int)rows, n, p, c, (int)T, ntiles, pools.ws_step)
   const bool split = p >= BM;
   // whole-chunk loads: c a multiple of two chunks, and a 128-row panel addressable with
   // 32-bit offsets (any pool size: the buffer resources are based at each tile's panels)

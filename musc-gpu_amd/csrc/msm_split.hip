@@ -78,14 +78,18 @@ constexpr int kBufferFlags = 0x00020000;     // buffer resource word 3 for raw b
 // Prepare: one wave per row.  norms[], scale[] and the image maxima exactly as
 // msm_norms_kernel; inv[] holds the epilogue's per-row scale of the split dot product.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void split_prepare_kernel(const float* __restrict__ z, int rows, int c, int nkb,
-                                                            int normalize, float* __restrict__ norms,
-                                                            float* __restrict__ inv, float* __restrict__ scale,
-                                                            _Float16* __restrict__ hl) {
+__global__ __launch_bounds__(256) void split_prepare_kernel(const float* __restrict__ z, int rows, int n, int c,
+                                                            int nkb, int normalize, Workspace w,
+                                                            _Float16* __restrict__ hl, size_t ws_step) {
   const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
   const long long row = (long long)blockIdx.x * (blockDim.x / kWave) + wave;
   if (row >= rows) return;
-  const float* src = z + row * (long long)c;
+  float* const norms = pool_ptr(w.norms, ws_step);
+  float* const inv = pool_ptr(w.inv, ws_step);
+  float* const scale = pool_ptr(w.scale, ws_step);
+  hl = pool_ptr(hl, ws_step);
+  fill_row_keys(pool_ptr(w.minbits, ws_step) + row * n, n, lane);
+  const float* src = z + (blockIdx.y * (long long)rows + row) * c;
   // A row of whole 32-channel pairs of blocks, up to 1024 channels (the pools' C), stays in
   // registers between its norm and its split (at most 4 float4 per lane, taken by the same
   // lanes in the same order as row_sumsq, so the same sum); otherwise the split reads the
@@ -212,7 +216,7 @@ __global__ __launch_bounds__(THREADS, 1) void split_pair_kernel(const _Float16* 
                                                                const float* __restrict__ norms,
                                                                const float* __restrict__ inv,
                                                                uint32_t* __restrict__ minbits, int rows, int n, int p,
-                                                               int nkb, int T, long long ntiles) {
+                                                               int nkb, int T, long long ntiles, size_t ws_step) {
   __shared__ __attribute__((aligned(16))) unsigned char smem[NSTAGE * kStageBytes];
   __shared__ __attribute__((aligned(16))) float s_rnorm[TM];
   __shared__ __attribute__((aligned(16))) float s_rinv[TM];
@@ -229,6 +233,10 @@ __global__ __launch_bounds__(THREADS, 1) void split_pair_kernel(const _Float16* 
   // no padding); a tile of one image only has no pair to score
   const bool simple = (row0 + TM <= rows) && (col0 + TM <= rows) && (rlast / p == rimg0) && (clast / p == cimg0);
   if (simple && rimg0 == cimg0) return;
+  hl = pool_ptr(hl, ws_step);  // this workgroup's pool
+  norms = pool_ptr(norms, ws_step);
+  inv = pool_ptr(inv, ws_step);
+  minbits = pool_ptr(minbits, ws_step);
 
   const int t = threadIdx.x;  // THREADS == TM: thread t merges tile row t and tile column t
   const int wave = t / kWave, lane = t % kWave;
@@ -747,7 +755,9 @@ inline _Float16* split_array(void* ws, long long n, long long p) {
   return reinterpret_cast<_Float16*>(static_cast<char*>(ws) + msm::workspace_bytes(n, p));
 }
 
-inline int validate(int n, int p, int c, void* ws, size_t ws_bytes) {
+size_t pool_workspace_bytes(long long n, long long p, int c) { return workspace_bytes(n, p, c); }
+
+int validate(int n, int p, int c, void* ws, size_t ws_bytes) {
   if (n < 2 || p < 1 || c < 1) return MUSC_ERR_INVALID_ARG;
   const long long rows = (long long)n * p;
   if (rows > (1LL << 30) || n > 4096) return MUSC_ERR_UNSUPPORTED;
@@ -758,16 +768,15 @@ inline int validate(int n, int p, int c, void* ws, size_t ws_bytes) {
   return MUSC_OK;
 }
 
-inline void run_prepare(const float* z, int n, int p, int c, int normalize, void* ws, hipStream_t s) {
+void run_prepare(const float* z, int n, int p, int c, int normalize, void* ws, const Pools& pools, hipStream_t s) {
   const long long rows = (long long)n * p;
   const Workspace w = carve(ws, n, p);
-  hipLaunchKernelGGL(split_prepare_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, z, (int)rows, c,
-                     nkb_of(c), normalize, w.norms, w.inv, w.scale, split_array(ws, n, p));
-  launch_image_max(w.norms, n, p, w.imgmax, s);
-  launch_fill_u32(w.minbits, (size_t)rows * n, kMinFill, s);
+  hipLaunchKernelGGL(split_prepare_kernel, dim3((unsigned)((rows + 3) / 4), pools.count), dim3(256), 0, s, z, (int)rows,
+                     n, c, nkb_of(c), normalize, w, split_array(ws, n, p), pools.ws_step);
+  launch_image_max(w.norms, n, p, w.imgmax, pools, s);
 }
 
-inline int run_pairs(int n, int p, int c, void* ws, hipStream_t s) {
+int run_pairs(int n, int p, int c, void* ws, const Pools& pools, hipStream_t s) {
   if (p < TM) return MUSC_ERR_UNSUPPORTED;  // the two-segment epilogue needs p >= 256
   const long long rows = (long long)n * p;
   const long long T = (rows + TM - 1) / TM;
@@ -775,8 +784,8 @@ inline int run_pairs(int n, int p, int c, void* ws, hipStream_t s) {
   const long long grid = (ntiles + kXcds - 1) / kXcds * kXcds;  // one workgroup per tile
   if (grid > 0x7fffffffLL) return MUSC_ERR_UNSUPPORTED;
   const Workspace w = carve(ws, n, p);
-  hipLaunchKernelGGL(split_pair_kernel, dim3((unsigned)grid), dim3(THREADS), 0, s, split_array(ws, n, p), w.norms,
-                     w.inv, w.minbits, (int)rows, n, p, nkb_of(c), (int)T, ntiles);
+  hipLaunchKernelGGL(split_pair_kernel, dim3((unsigned)grid, pools.count), dim3(THREADS), 0, s, split_array(ws, n, p),
+                     w.norms, w.inv, w.minbits, (int)rows, n, p, nkb_of(c), (int)T, ntiles, pools.ws_step);
   return check_launch();
 }
 
@@ -798,7 +807,7 @@ extern "C" int musc_msm_split_prepare_f32(const float* z, int n, int p, int c, i
   if (rc) return rc;
   if (!z || (flags & ~MUSC_MSM_NORMALIZE_ROWS)) return MUSC_ERR_INVALID_ARG;
   if ((c & 3) == 0 && (reinterpret_cast<uintptr_t>(z) & 15) != 0) return MUSC_ERR_INVALID_ARG;
-  msm::split::run_prepare(z, n, p, c, (flags & MUSC_MSM_NORMALIZE_ROWS) ? 1 : 0, workspace, stream);
+  msm::split::run_prepare(z, n, p, c, (flags & MUSC_MSM_NORMALIZE_ROWS) ? 1 : 0, workspace, msm::kOnePool, stream);
   return check_launch();
 }
 
@@ -806,7 +815,7 @@ extern "C" int musc_msm_split_pair_minima(int n, int p, int c, void* workspace, 
                                           hipStream_t stream) {
   int rc = msm::split::validate(n, p, c, workspace, workspace_bytes);
   if (rc) return rc;
-  return msm::split::run_pairs(n, p, c, workspace, stream);
+  return msm::split::run_pairs(n, p, c, workspace, msm::kOnePool, stream);
 }
 
 extern "C" int musc_msm_split_scores_f32(const float* z, int n, int p, int c, int rank_lo, int rank_hi, int flags,
@@ -818,11 +827,11 @@ extern "C" int musc_msm_split_scores_f32(const float* z, int n, int p, int c, in
   if (flags & ~MUSC_MSM_NORMALIZE_ROWS) return MUSC_ERR_INVALID_ARG;
   if ((c & 3) == 0 && (reinterpret_cast<uintptr_t>(z) & 15) != 0) return MUSC_ERR_INVALID_ARG;
   if (p < msm::split::TM) return MUSC_ERR_UNSUPPORTED;
-  msm::split::run_prepare(z, n, p, c, (flags & MUSC_MSM_NORMALIZE_ROWS) ? 1 : 0, workspace, stream);
-  rc = msm::split::run_pairs(n, p, c, workspace, stream);
+  msm::split::run_prepare(z, n, p, c, (flags & MUSC_MSM_NORMALIZE_ROWS) ? 1 : 0, workspace, msm::kOnePool, stream);
+  rc = msm::split::run_pairs(n, p, c, workspace, msm::kOnePool, stream);
   if (rc) return rc;
   const msm::Workspace w = msm::carve(workspace, n, p);
-  rc = msm::run_refine(z, n, p, c, w, stream);
+  rc = msm::run_refine(z, n, p, c, w, msm::kOnePool, stream);
   if (rc) return rc;
-  return msm::run_rank(n, p, rank_lo, rank_hi, scores, w, stream);
+  return msm::run_rank(n, p, rank_lo, rank_hi, scores, w, msm::kOnePool, stream);
 }

@@ -39,6 +39,7 @@ LNAMD_L2NORM = 1
 LNAMD_STATS_READY = 2
 LNAMD_RAW_SUMS = 4
 MSM_NORMALIZE_ROWS = 1
+MSM_ENGINES = {'fp32': 0, 'split16': 1}
 
 # Every symbol include/musc_hip.h declares, with its ctypes signature.
 _vp, _i, _f, _sz, _ll = ctypes.c_void_p, ctypes.c_int, ctypes.c_float, ctypes.c_size_t, ctypes.c_longlong
@@ -58,6 +59,8 @@ SIGNATURES = {
     'musc_msm_split_prepare_f32': (_i, [_vp, _i, _i, _i, _i, _vp, _sz, _vp]),
     'musc_msm_split_pair_minima': (_i, [_i, _i, _i, _vp, _sz, _vp]),
     'musc_msm_split_scores_f32': (_i, [_vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _sz, _vp]),
+    'musc_msm_pools_workspace_bytes': (_i, [_i, _i, _i, _i, _i, ctypes.POINTER(_sz)]),
+    'musc_msm_pools_scores_f32': (_i, [_vp, _i, _i, _i, _i, _i, _i, _i, _i, _vp, _vp, _sz, _vp]),
     'musc_lnamd_workspace_bytes': (_i, [_i, _i, ctypes.POINTER(_sz)]),
     'musc_lnamd_f32': (_i, [_vp, _i, _i, _i, _i, _i, _i, _vp, _i, _f, _i, _vp, _i, _vp, _sz, _vp]),
     'musc_lnamd_pooled_f32': (_i, [_vp, _i, _i, _i, _i, _i, _i, _vp, _i, _f, _i, _i, _vp, _i, _vp, _sz, _vp]),

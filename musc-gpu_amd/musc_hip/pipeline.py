@@ -17,7 +17,8 @@ the LayerNorm scale and the 1/r^2 of the box mean cancel in the L2
 normalisation, which the MSM applies to each row on the fly
 (MUSC_MSM_NORMALIZE_ROWS: its norms pass computes 1/||row|| and the pair
 kernel's epilogue scales each dot product), so no pass over the 5.6 GB exists
-just to normalise.  The R*L MSM calls reuse one workspace and write into one
+just to normalise.  The R*L pools are scored a few per launch (one workspace of at
+most 256 MiB, or one pool's) into one
 (R, L, N, P) float64 score tensor, which the epilogue kernel reduces, upsamples
 and maximises.  Everything is asynchronous on torch's current stream.
 """
@@ -28,6 +29,11 @@ import torch
 from . import _MSM_hip, _epilogue_hip, _lnamd_hip
 from ._RsCIN_hip import RsCIN
 from . import _runtime as rt
+
+
+# Workspace of one launch over several pools: the reference's own scratch cap
+# (models/modules/_MSM_gpu.py:11).  Larger pools are scored one at a time.
+POOLS_WORKSPACE = 256 << 20
 
 
 def lnamd_pools(tokens: list[torch.Tensor], r_list: list[int], pool_grid: int | None = None) -> torch.Tensor:
@@ -47,12 +53,13 @@ def msm_all(pools: torch.Tensor, topmin_min: float = 0, topmin_max: float = 0.3,
             rank_events: list | None = None, refine_events: list | None = None) -> torch.Tensor:
     """(R, L, N, P) float64 MSM maps of every (radius, layer) pool.
 
-    Runs the four MSM stages explicitly (prepare, pair minima, cancellation
-    refinement, rank) so that a caller can pass `pair_events`, a list that receives one (start, end)
+    The pools go through one launch per MSM stage together, as many at a time as
+    fit POOLS_WORKSPACE.  With `pair_events`, a list that receives one (start, end)
     torch.cuda.Event pair recorded around each pair-minima kernel on the stream
     it runs on (`rank_events` and `refine_events` the same around each rank and
-    cancellation-refinement kernel).  `engine` selects how the dot products are
-    formed ('fp32' or 'split16', see _MSM_hip).
+    cancellation-refinement kernel), the four stages (prepare, pair minima,
+    cancellation refinement, rank) run explicitly, pool by pool.  `engine` selects how
+    the dot products are formed ('fp32' or 'split16', see _MSM_hip).
     """
     rt.require_device_tensor(pools, 'pools')
     if pools.ndim != 5 or pools.dtype != torch.float32 or not pools.is_contiguous():
@@ -67,8 +74,19 @@ def msm_all(pools: torch.Tensor, topmin_min: float = 0, topmin_max: float = 0.3,
     split = engine == 'split16'
     with torch.cuda.device(pools.device):
         scores = torch.empty((r, l, n, p), dtype=torch.float64, device=pools.device)
-        ws = rt.workspace(_MSM_hip.workspace_bytes(n, p, c, engine), pools.device)
+        per_pool = _MSM_hip.workspace_bytes(n, p, c, engine)
         s = rt.stream(pools.device)
+        if pair_events is None and rank_events is None and refine_events is None:
+            group = min(r * l, max(1, POOLS_WORKSPACE // per_pool))
+            ws = rt.workspace(group * per_pool, pools.device)
+            z_step, s_step = n * p * c * 4, n * p * 8
+            for k in range(0, r * l, group):
+                rt.check(lib.musc_msm_pools_scores_f32(pools.data_ptr() + k * z_step, min(group, r * l - k), n, p, c, a,
+                                                       b, flags, rt.MSM_ENGINES[engine],
+                                                       scores.data_ptr() + k * s_step, ws.data_ptr(), ws.numel(), s),
+                         'musc_msm_pools_scores_f32')
+            return scores
+        ws = rt.workspace(per_pool, pools.device)
         for ri in range(r):
             for li in range(l):
                 z = pools[ri, li]

@@ -181,3 +181,23 @@ def test_preprocess_workspace_and_argument_errors(lib):
     assert lib.musc_preprocess_u8(None, 1, 10, 10, 5, 5, m, m, fake, fake, big, None) == 1001
     assert lib.musc_preprocess_u8(fake, 1, 10, 10, 5, 5, m, s0, fake, fake, big, None) == 1001   # zero std
     assert lib.musc_preprocess_u8(fake, 1, 10, 10, 5, 5, m, m, fake, fake, ctypes.c_size_t(8), None) == 1002
+
+
+def test_msm_pools_argument_errors(lib):
+    one, many = ctypes.c_size_t(), ctypes.c_size_t()
+    for engine, name in ((0, 'musc_msm_workspace_bytes'), (1, 'musc_msm_split_workspace_bytes')):
+        assert getattr(lib, name)(5, 300, 33, ctypes.byref(one)) == 0
+        assert lib.musc_msm_pools_workspace_bytes(7, 5, 300, 33, engine, ctypes.byref(many)) == 0
+        assert many.value == 7 * one.value and one.value % 256 == 0
+    assert lib.musc_msm_pools_workspace_bytes(0, 5, 300, 33, 0, ctypes.byref(many)) == 1001
+    assert lib.musc_msm_pools_workspace_bytes(2, 5, 300, 33, 2, ctypes.byref(many)) == 1001
+    fake, big = ctypes.c_void_p(256), ctypes.c_size_t(1 << 40)
+
+    def call(z=fake, pools=2, n=8, p=300, c=16, a=0, b=2, flags=0, engine=0, ws=fake, size=big):
+        return lib.musc_msm_pools_scores_f32(z, pools, n, p, c, a, b, flags, engine, fake, ws, size, None)
+
+    assert call(z=None) == 1001 and call(pools=0) == 1001 and call(engine=2) == 1001 and call(flags=4) == 1001
+    assert call(a=2) == 1001 and call(b=8) == 1001 and call(ws=ctypes.c_void_p(264)) == 1001
+    assert call(pools=70000) == 1003 and call(engine=1, p=100) == 1003 and call(n=5000, p=1) == 1003
+    assert lib.musc_msm_workspace_bytes(8, 300, 16, ctypes.byref(one)) == 0
+    assert call(size=ctypes.c_size_t(2 * one.value - 1)) == 1002

@@ -70,3 +70,25 @@ def test_config2_full_size_sampled_images(device):
     err_i = (img[list(picks)] - ref_img).abs().max().item()
     print(f'config2 sampled maps err {err_m:.3e}, image score err {err_i:.3e}', flush=True)
     assert err_m <= ATOL and err_i <= ATOL
+
+
+@pytest.mark.parametrize('engine,r,l,n,p,c', [('fp32', 2, 2, 8, 144, 256), ('fp32', 1, 3, 3, 1, 4), ('fp32', 3, 1, 5, 130, 33),
+                                              ('fp32', 1, 2, 200, 9, 64), ('split16', 2, 2, 4, 289, 96),
+                                              ('split16', 1, 5, 3, 256, 20)])
+@pytest.mark.parametrize('group', [1, 2, 100])
+def test_pools_in_one_launch_match_pool_by_pool(device, monkeypatch, engine, r, l, n, p, c, group):
+    # several pools per launch (all of them, two at a time with a rest, one) against the stages run
+    # pool by pool: the same kernels on the same rows, so the same bits; one pool holds a duplicated
+    # image (refined minima) and one a NaN row
+    from musc_hip import _MSM_hip
+    g = torch.Generator().manual_seed(n * p + c)
+    z = torch.randn((r, l, n, p, c), generator=g)
+    z[0, 0, n - 1] = z[0, 0, 0]
+    z[r - 1, l - 1, 1, 0] = float('nan')
+    z = z.to(device)
+    monkeypatch.setattr(pipeline, 'POOLS_WORKSPACE', group * _MSM_hip.workspace_bytes(n, p, c, engine))
+    window = dict(topmin_min=0, topmin_max=max(1, n // 3))
+    for normalize in (True, False):
+        got = pipeline.msm_all(z, normalize_rows=normalize, engine=engine, **window)
+        ref = pipeline.msm_all(z, normalize_rows=normalize, engine=engine, pair_events=[], **window)
+        assert torch.equal(got.view(torch.int64), ref.view(torch.int64))
