@@ -1,7 +1,8 @@
 // fp32 MFMA pairwise minima of the mutual scoring module (MSM) for gfx950.
 //
 // msm_pair_min_kernel: the whole pool is one (n*p) x (n*p) Gram matrix.  Only the
-// upper triangle of 128x128 tiles is computed, on fp32 MFMA (v_mfma_f32_32x32x2f32),
+// upper triangle of its 128x128 tiles (64x64 for small pools) is computed, on fp32 MFMA
+// (v_mfma_f32_32x32x2f32),
 // so each unordered patch pair's dot product is formed once.  The epilogue turns dots
 // into squared distances ||a||^2 + ||b||^2 - 2 a.b (clamped at 0, as torch.cdist's
 // matmul path does; models/modules/_MSM.py:16-17), masks same-image pairs, and
@@ -16,21 +17,23 @@
 namespace musc {
 namespace msm {
 
-constexpr int BM = 128;          // tile rows (query patches)
-constexpr int BN = 128;          // tile columns (reference patches)
+// kW: 32 x 32 MFMA blocks per wave and dimension.  kW = 2 is the 128 x 128 tile; kW = 1 a
+// 64 x 64 tile of the same four waves, for pools whose 128-tiles leave most CUs idle.
+constexpr int tile_of(int kW) { return 64 * kW; }
 constexpr int BK = 16;           // K chunk (channels) per pipeline stage: the double-buffered
                                  // stage is 40 KB of LDS, so three workgroups share a CU
                                  // (three waves per SIMD cover each other's epilogues and barriers)
 constexpr int PITCH = BK;        // LDS row pitch in floats for staged operands (64 bytes)
-constexpr int EPITCH = BN + 1;   // LDS row pitch of the epilogue distance tile
-constexpr int THREADS = 256;     // 4 waves, each owns a 64x64 sub-tile
-constexpr int kRowsPerPass = THREADS / (BK / 4);  // rows one 16-byte load per thread covers
-constexpr int kPasses = BM / kRowsPerPass;         // such loads per thread per staged operand
+constexpr int THREADS = 256;     // 4 waves, each owns a quarter of the tile
+constexpr int kRowsPerPass = THREADS / (BK / 4);  // rows one 16-byte load per thread covers (64)
 
 static_assert(BK == 16 && kRowsPerPass % 16 == 0, "the segment swizzle assumes 4 segments per row");
-constexpr int kStageFloats = 2 * (BM + BN) * PITCH;       // double-buffered A and B
-constexpr int kEpiFloats = BM * EPITCH;
-constexpr int kSmemFloats = kStageFloats > kEpiFloats ? kStageFloats : kEpiFloats;
+constexpr int stage_floats(int kW) { return 2 * 2 * tile_of(kW) * PITCH; }  // double-buffered A and B
+// the small-p epilogue's distance tile (pitch tile + 1) shares the staging buffers
+constexpr int smem_floats(int kW, bool split) {
+  const int epi = tile_of(kW) * (tile_of(kW) + 1);
+  return split || stage_floats(kW) > epi ? stage_floats(kW) : epi;
+}
 constexpr int kBufferFlags = 0x00020000;  // buffer resource word 3 for raw byte-addressed loads
 
 // ---------------------------------------------------------------------------
@@ -43,7 +46,7 @@ typedef float stage4 __attribute__((ext_vector_type(4)));
 
 // Channel-masked operand loads: kLoad 1 = 16-byte loads (c % 4 == 0), 0 = scalar loads.
 // (kLoad 2, whole chunks through a buffer resource, is in the kernel.)
-template <int kLoad>
+template <int kLoad, int kPasses>
 __device__ inline void load_chunk(const float* __restrict__ z, int rows, int c, int row0, int k0,
                                   stage4 (&reg)[kPasses]) {
   static_assert(kLoad == 0 || kLoad == 1, "whole-chunk loads are issued by the kernel");
@@ -77,6 +80,7 @@ __device__ inline void load_chunk(const float* __restrict__ z, int rows, int c, 
 // of a 64-byte pitch, or r and r + 3 of an 80-byte one, share banks).
 __device__ inline int seg_swizzle(int row) { return (row >> 2) & 3; }
 
+template <int kPasses>
 __device__ inline void store_chunk(float* __restrict__ dst, const stage4 (&reg)[kPasses]) {
   const int t = threadIdx.x;
   const int lrow = t / (BK / 4);
@@ -87,14 +91,18 @@ __device__ inline void store_chunk(float* __restrict__ dst, const stage4 (&reg)[
     *reinterpret_cast<stage4*>(dst + (lrow + kRowsPerPass * i) * PITCH + lk) = reg[i];
 }
 
-// kSplit (p >= BM): a 128-row or 128-column range holds at most one image boundary,
+// kSplit (p >= the tile): a tile's row or column range holds at most one image boundary,
 // so tiles straddling a boundary reduce in registers too, with two image segments
-// per dimension; otherwise (small p) they go through the LDS epilogue.
-template <int kLoad, bool kSplit>
-__global__ __launch_bounds__(THREADS, kSplit ? 3 : 2) void msm_pair_min_kernel(
+// per dimension; otherwise (p < 64) they go through the LDS epilogue.
+template <int kLoad, bool kSplit, int kW>
+__global__ __launch_bounds__(THREADS, kSplit || kW == 1 ? 3 : 2) void msm_pair_min_kernel(
     const float* __restrict__ z, const float* __restrict__ norms, const float* __restrict__ inv,
     uint32_t* __restrict__ minbits, int rows, int n, int p, int c, int T, long long ntiles, size_t ws_step) {
-  __shared__ __attribute__((aligned(16))) float smem[kSplit ? kStageFloats : kSmemFloats];
+  constexpr int BM = tile_of(kW), BN = BM;    // tile rows (query patches), columns (reference patches)
+  constexpr int SW = 32 * kW;                 // rows and columns of a wave's sub-tile
+  constexpr int EPITCH = BN + 1;              // LDS row pitch of the epilogue distance tile
+  constexpr int kPasses = BM / kRowsPerPass;  // 16-byte loads per thread per staged operand
+  __shared__ __attribute__((aligned(16))) float smem[smem_floats(kW, kSplit)];
   __shared__ __attribute__((aligned(16))) float s_rnorm[BM];
   __shared__ __attribute__((aligned(16))) float s_cnorm[BN];
   __shared__ __attribute__((aligned(16))) float s_rinv[BM];   // -2 x row scale (the scale is 1 unless normalising)
@@ -123,7 +131,7 @@ __global__ __launch_bounds__(THREADS, kSplit ? 3 : 2) void msm_pair_min_kernel(
     s_rnorm[t] = r < rows ? norms[r] : 0.f;
     s_rinv[t] = r < rows ? -2.f * inv[r] : 0.f;  // exact: a power-of-two factor
     s_rimg[t] = r < rows ? r / p : n;  // n marks "no image" (padding)
-  } else {
+  } else if (t < BM + BN) {
     const int cc = col0 + (t - BM);
     s_cnorm[t - BM] = cc < rows ? norms[cc] : 0.f;
     s_cinv[t - BM] = cc < rows ? inv[cc] : 0.f;
@@ -134,11 +142,11 @@ __global__ __launch_bounds__(THREADS, kSplit ? 3 : 2) void msm_pair_min_kernel(
   const int wm = wave >> 1, wn = wave & 1;
   const int lr = lane & 31, lh = lane >> 5;
 
-  floatx16 acc[2][2];
+  floatx16 acc[kW][kW];
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+  for (int a = 0; a < kW; ++a)
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+    for (int b = 0; b < kW; ++b)
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.f;
 
@@ -175,7 +183,7 @@ __global__ __launch_bounds__(THREADS, kSplit ? 3 : 2) void msm_pair_min_kernel(
                                                                                   (int)(rowsA ? voffA[i] : voffB[i]),
                                                                                   k0 * 4, 0));
     } else {
-      load_chunk<kLoad>(z, rows, c, rowsA ? row0 : col0, k0, reg);
+      load_chunk<kLoad, kPasses>(z, rows, c, rowsA ? row0 : col0, k0, reg);
     }
   };
   // An even number of chunks, so the K loop below leaves only at its end: an exit
@@ -197,26 +205,28 @@ __global__ __launch_bounds__(THREADS, kSplit ? 3 : 2) void msm_pair_min_kernel(
   load(false, min(2, nk - 1) * BK, rb0);
   __syncthreads();
 
-  // lane (lr, lh) reads segments lh and lh + 2 of rows wm*64 + lr (+ 32) and wn*64 + lr
+  // lane (lr, lh) reads segments lh and lh + 2 of rows wm*SW + lr (+ 32) and wn*SW + lr
   // (+ 32): the row offsets are multiples of 16, so the swizzle is that of lr
   const int seg_off[2] = {4 * (lh ^ seg_swizzle(lr)), 4 * ((lh + 2) ^ seg_swizzle(lr))};
   auto compute = [&](int buf) {
-    const float* A = smem + buf * kStage + (wm * 64 + lr) * PITCH;
-    const float* B = smem + buf * kStage + BM * PITCH + (wn * 64 + lr) * PITCH;
+    const float* A = smem + buf * kStage + (wm * SW + lr) * PITCH;
+    const float* B = smem + buf * kStage + BM * PITCH + (wn * SW + lr) * PITCH;
 #pragma unroll
     for (int s = 0; s < BK / 8; ++s) {
-      const float4 a0 = *reinterpret_cast<const float4*>(A + seg_off[s]);
-      const float4 a1 = *reinterpret_cast<const float4*>(A + 32 * PITCH + seg_off[s]);
-      const float4 b0 = *reinterpret_cast<const float4*>(B + seg_off[s]);
-      const float4 b1 = *reinterpret_cast<const float4*>(B + 32 * PITCH + seg_off[s]);
-      const float av[2][4] = {{a0.x, a0.y, a0.z, a0.w}, {a1.x, a1.y, a1.z, a1.w}};
-      const float bv[2][4] = {{b0.x, b0.y, b0.z, b0.w}, {b1.x, b1.y, b1.z, b1.w}};
+      float av[kW][4], bv[kW][4];
+#pragma unroll
+      for (int i = 0; i < kW; ++i) {
+        const float4 a = *reinterpret_cast<const float4*>(A + 32 * i * PITCH + seg_off[s]);
+        const float4 b = *reinterpret_cast<const float4*>(B + 32 * i * PITCH + seg_off[s]);
+        av[i][0] = a.x, av[i][1] = a.y, av[i][2] = a.z, av[i][3] = a.w;
+        bv[i][0] = b.x, bv[i][1] = b.y, bv[i][2] = b.z, bv[i][3] = b.w;
+      }
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
+        for (int mb = 0; mb < kW; ++mb)
 #pragma unroll
-          for (int nb = 0; nb < 2; ++nb)
+          for (int nb = 0; nb < kW; ++nb)
             acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[mb][e], bv[nb][e], acc[mb][nb], 0, 0, 0);
     }
   };
@@ -239,59 +249,67 @@ __global__ __launch_bounds__(THREADS, kSplit ? 3 : 2) void msm_pair_min_kernel(
     __syncthreads();
   }
 
-  if (simple) {
-    // Register epilogue.  Lane (lr, lh) of wave (wm, wn) holds, for mb, nb in {0,1} and
-    // v in 0..15, the dot of tile row wm*64 + mb*32 + (v/4)*8 + lh*4 + v%4 with tile
-    // column wn*64 + nb*32 + lr.
-    float d2[2][2][16];
+  // the reduced column this lane stores: of the column blocks' 32 columns, half lh keeps block lh
+  const int ccol = (kW == 2 ? lh * 32 : 0) + lr;
+  // one block of rows: transpose_min32's upper 16 items are empty (lanes 16-31 hold none)
+  auto no_items = [](float (&rv)[32]) {
 #pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
+    for (int v = 16; v < 32; ++v) rv[v] = __int_as_float(kInfBits);
+  };
+  if (simple) {
+    // Register epilogue.  Lane (lr, lh) of wave (wm, wn) holds, for mb, nb < kW and
+    // v in 0..15, the dot of tile row wm*SW + mb*32 + (v/4)*8 + lh*4 + v%4 with tile
+    // column wn*SW + nb*32 + lr.
+    float d2[kW][kW][16];
+#pragma unroll
+    for (int mb = 0; mb < kW; ++mb)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const float4 rn = *reinterpret_cast<const float4*>(&s_rnorm[wm * 64 + mb * 32 + g * 8 + lh * 4]);
-        const float4 ri = *reinterpret_cast<const float4*>(&s_rinv[wm * 64 + mb * 32 + g * 8 + lh * 4]);
+        const float4 rn = *reinterpret_cast<const float4*>(&s_rnorm[wm * SW + mb * 32 + g * 8 + lh * 4]);
+        const float4 ri = *reinterpret_cast<const float4*>(&s_rinv[wm * SW + mb * 32 + g * 8 + lh * 4]);
         const float rv[4] = {rn.x, rn.y, rn.z, rn.w};
         const float rs[4] = {ri.x, ri.y, ri.z, ri.w};
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb) {
-          const float cn = s_cnorm[wn * 64 + nb * 32 + lr];
-          const float ci = s_cinv[wn * 64 + nb * 32 + lr];
+        for (int nb = 0; nb < kW; ++nb) {
+          const float cn = s_cnorm[wn * SW + nb * 32 + lr];
+          const float ci = s_cinv[wn * SW + nb * 32 + lr];
 #pragma unroll
           for (int e = 0; e < 4; ++e)  // clamped at 0 after the minima: max(., 0) commutes with min
             d2[mb][nb][g * 4 + e] = fmaf(rs[e] * ci, acc[mb][nb][g * 4 + e], rv[e] + cn);
         }
       }
     // column minima over this wave's 64 rows: in-lane, then across the two lane halves
-    float cmin[2];
+    float cmin[kW];
 #pragma unroll
-    for (int nb = 0; nb < 2; ++nb) {
+    for (int nb = 0; nb < kW; ++nb) {
       float m = d2[0][nb][0];
 #pragma unroll
-      for (int mb = 0; mb < 2; ++mb)
+      for (int mb = 0; mb < kW; ++mb)
 #pragma unroll
         for (int v = 0; v < 16; ++v) m = nmin(m, d2[mb][nb][v]);
       cmin[nb] = m;
     }
     // half lh keeps column block nb = lh, with the other half's minimum for it
-    cmin[0] = halves_min2(cmin[0], cmin[1]);
+    cmin[0] = halves_min2(cmin[0], cmin[kW - 1]);
     // row minima over this wave's 64 columns: min over nb in-lane, then a transposing
     // butterfly over the 32 lanes of each half (31 exchanges); lane lr ends with the
     // minimum of value index k = lr, i.e. row (lr/16)*32 + ((lr%16)/4)*8 + lh*4 + lr%4.
     float rv[32];
 #pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
+    for (int mb = 0; mb < kW; ++mb)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) rv[mb * 16 + v] = nmin(d2[mb][0][v], d2[mb][1][v]);
+      for (int v = 0; v < 16; ++v) rv[mb * 16 + v] = nmin(d2[mb][0][v], d2[mb][kW - 1][v]);
+    if constexpr (kW == 1) no_items(rv);
     transpose_min32(rv, lr);
     __syncthreads();  // operand buffers are no longer read
     float* s_cmin = smem;             // [2 (wm)][BN]
     float* s_rmin = smem + 2 * BN;    // [2 (wn)][BM]
-    s_cmin[wm * BN + wn * 64 + lh * 32 + lr] = cmin[0];
-    s_rmin[wn * BM + wm * 64 + (lr >> 4) * 32 + ((lr & 15) >> 2) * 8 + lh * 4 + (lr & 3)] = rv[0];
+    s_cmin[wm * BN + wn * SW + ccol] = cmin[0];
+    if (kW == 2 || lr < 16) s_rmin[wn * BM + wm * SW + transposed_row(lr, lh)] = rv[0];
     __syncthreads();
     if (t < BM) {
       atomicMin(minbits + (long long)(row0 + t) * n + cimg0, min_key(nmin(s_rmin[t], s_rmin[BM + t])));
-    } else {
+    } else if (t < BM + BN) {
       const int j = t - BM;
       atomicMin(minbits + (long long)(col0 + j) * n + rimg0, min_key(nmin(s_cmin[j], s_cmin[BN + j])));
     }
@@ -299,7 +317,7 @@ __global__ __launch_bounds__(THREADS, kSplit ? 3 : 2) void msm_pair_min_kernel(
   }
 
   if constexpr (kSplit) {
-    // Two-segment register epilogue (P >= 128, so a 128-row or 128-column range holds
+    // Two-segment register epilogue (P >= the tile, so a tile's row or column range holds
     // at most one image boundary).  Tile rows [0, rsplit) belong to image rA, rows
     // [rsplit, BM) to image rA + 1 or to the padding (image n); columns likewise with
     // csplit and cA.  Whether a pair is masked (same image, or padding) depends only
@@ -315,51 +333,51 @@ __global__ __launch_bounds__(THREADS, kSplit ? 3 : 2) void msm_pair_min_kernel(
     const int cBimg = col0 + csplit < rows ? cA + 1 : n;
     const bool mAA = rA == cA, mAB = cBimg == n || rA == cBimg;
     const bool mBA = rBimg == n || rBimg == cA, mBB = rBimg == n || cBimg == n || rBimg == cBimg;
-    float d2[2][2][16];
+    float d2[kW][kW][16];
 #pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
+    for (int mb = 0; mb < kW; ++mb)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const int i0 = wm * 64 + mb * 32 + g * 8 + lh * 4;
+        const int i0 = wm * SW + mb * 32 + g * 8 + lh * 4;
         const float4 rn = *reinterpret_cast<const float4*>(&s_rnorm[i0]);
         const float4 ri = *reinterpret_cast<const float4*>(&s_rinv[i0]);
         const float rv[4] = {rn.x, rn.y, rn.z, rn.w};
         const float rs[4] = {ri.x, ri.y, ri.z, ri.w};
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb) {
-          const float cn = s_cnorm[wn * 64 + nb * 32 + lr];
-          const float ci = s_cinv[wn * 64 + nb * 32 + lr];
+        for (int nb = 0; nb < kW; ++nb) {
+          const float cn = s_cnorm[wn * SW + nb * 32 + lr];
+          const float ci = s_cinv[wn * SW + nb * 32 + lr];
 #pragma unroll
           for (int e = 0; e < 4; ++e)  // clamped at 0 after the minima
             d2[mb][nb][g * 4 + e] = fmaf(rs[e] * ci, acc[mb][nb][g * 4 + e], rv[e] + cn);
         }
       }
     // column minima over this wave's 64 rows, per row segment, then across lane halves
-    const int wr0 = wm * 64, wc0 = wn * 64;
-    float cminA[2], cminB[2];
-    if (rsplit >= wr0 + 64 || rsplit <= wr0) {
-      float m[2];
+    const int wr0 = wm * SW, wc0 = wn * SW;
+    float cminA[kW], cminB[kW];
+    if (rsplit >= wr0 + SW || rsplit <= wr0) {
+      float m[kW];
 #pragma unroll
-      for (int nb = 0; nb < 2; ++nb) {
+      for (int nb = 0; nb < kW; ++nb) {
         float x = d2[0][nb][0];
 #pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
+        for (int mb = 0; mb < kW; ++mb)
 #pragma unroll
           for (int v = 0; v < 16; ++v) x = nmin(x, d2[mb][nb][v]);
         m[nb] = x;
       }
       const bool inA = rsplit > wr0;
 #pragma unroll
-      for (int nb = 0; nb < 2; ++nb) {
+      for (int nb = 0; nb < kW; ++nb) {
         cminA[nb] = inA ? m[nb] : inf;
         cminB[nb] = inA ? inf : m[nb];
       }
     } else {
 #pragma unroll
-      for (int nb = 0; nb < 2; ++nb) {
+      for (int nb = 0; nb < kW; ++nb) {
         float a = inf, b = inf;
 #pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
+        for (int mb = 0; mb < kW; ++mb)
 #pragma unroll
           for (int v = 0; v < 16; ++v) {
             const bool inB = wr0 + mb * 32 + (v >> 2) * 8 + lh * 4 + (v & 3) >= rsplit;
@@ -370,48 +388,51 @@ __global__ __launch_bounds__(THREADS, kSplit ? 3 : 2) void msm_pair_min_kernel(
         cminB[nb] = b;
       }
     }
-    float colA = halves_min2(cminA[0], cminA[1]);  // column wc0 + lh * 32 + lr
-    float colB = halves_min2(cminB[0], cminB[1]);
+    float colA = halves_min2(cminA[0], cminA[kW - 1]);  // column wc0 + ccol
+    float colB = halves_min2(cminB[0], cminB[kW - 1]);
     {
-      const bool colInB = wc0 + lh * 32 + lr >= csplit;
+      const bool colInB = wc0 + ccol >= csplit;
       if (colInB ? mAB : mAA) colA = inf;
       if (colInB ? mBB : mBA) colB = inf;
     }
     // row minima over this wave's 64 columns, per column segment: transposing
     // butterflies as in the single-segment path, two when the boundary falls inside
     float rowminA, rowminB;
-    if (csplit >= wc0 + 64 || csplit <= wc0) {
+    if (csplit >= wc0 + SW || csplit <= wc0) {
       float rv[32];
 #pragma unroll
-      for (int mb = 0; mb < 2; ++mb)
+      for (int mb = 0; mb < kW; ++mb)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) rv[mb * 16 + v] = nmin(d2[mb][0][v], d2[mb][1][v]);
+        for (int v = 0; v < 16; ++v) rv[mb * 16 + v] = nmin(d2[mb][0][v], d2[mb][kW - 1][v]);
+      if constexpr (kW == 1) no_items(rv);
       const float m = transpose_min32(rv, lr);
       const bool inA = csplit > wc0;
       rowminA = inA ? m : inf;
       rowminB = inA ? inf : m;
     } else {
-      const bool colB0 = wc0 + lr >= csplit, colB1 = wc0 + 32 + lr >= csplit;
+      const bool colB0 = wc0 + lr >= csplit, colB1 = wc0 + 32 * (kW - 1) + lr >= csplit;
       {
         float rv[32];
 #pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
+        for (int mb = 0; mb < kW; ++mb)
 #pragma unroll
           for (int v = 0; v < 16; ++v)
-            rv[mb * 16 + v] = nmin(colB0 ? inf : d2[mb][0][v], colB1 ? inf : d2[mb][1][v]);
+            rv[mb * 16 + v] = nmin(colB0 ? inf : d2[mb][0][v], colB1 ? inf : d2[mb][kW - 1][v]);
+        if constexpr (kW == 1) no_items(rv);
         rowminA = transpose_min32(rv, lr);
       }
       {
         float rv[32];
 #pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
+        for (int mb = 0; mb < kW; ++mb)
 #pragma unroll
           for (int v = 0; v < 16; ++v)
-            rv[mb * 16 + v] = nmin(colB0 ? d2[mb][0][v] : inf, colB1 ? d2[mb][1][v] : inf);
+            rv[mb * 16 + v] = nmin(colB0 ? d2[mb][0][v] : inf, colB1 ? d2[mb][kW - 1][v] : inf);
+        if constexpr (kW == 1) no_items(rv);
         rowminB = transpose_min32(rv, lr);
       }
     }
-    const int rk = wm * 64 + transposed_row(lr, lh);
+    const int rk = wm * SW + transposed_row(lr, lh);
     {
       const bool rowInB = rk >= rsplit;
       if (rowInB ? mBA : mAA) rowminA = inf;
@@ -422,10 +443,12 @@ __global__ __launch_bounds__(THREADS, kSplit ? 3 : 2) void msm_pair_min_kernel(
     float* s_cminB = smem + 2 * BN;
     float* s_rminA = smem + 4 * BN;   // [2 (wn)][BM]
     float* s_rminB = smem + 4 * BN + 2 * BM;
-    s_cminA[wm * BN + wn * 64 + lh * 32 + lr] = colA;
-    s_cminB[wm * BN + wn * 64 + lh * 32 + lr] = colB;
-    s_rminA[wn * BM + rk] = rowminA;
-    s_rminB[wn * BM + rk] = rowminB;
+    s_cminA[wm * BN + wn * SW + ccol] = colA;
+    s_cminB[wm * BN + wn * SW + ccol] = colB;
+    if (kW == 2 || lr < 16) {
+      s_rminA[wn * BM + rk] = rowminA;
+      s_rminB[wn * BM + rk] = rowminB;
+    }
     __syncthreads();
     if (t < BM) {
       const int r = row0 + t;
@@ -437,7 +460,7 @@ __global__ __launch_bounds__(THREADS, kSplit ? 3 : 2) void msm_pair_min_kernel(
         if (a != inf) atomicMin(minbits + (long long)r * n + cA, min_key(a));
         if (b != inf) atomicMin(minbits + (long long)r * n + cA + 1, min_key(b));
       }
-    } else {
+    } else if (t < BM + BN) {
       const int j = t - BM;
       const int cc = col0 + j;
       if (cc < rows) {
@@ -452,16 +475,16 @@ __global__ __launch_bounds__(THREADS, kSplit ? 3 : 2) void msm_pair_min_kernel(
   // Epilogue: squared distances into LDS (the operand buffers are free now).
   float* E = smem;
 #pragma unroll
-  for (int mb = 0; mb < 2; ++mb)
+  for (int mb = 0; mb < kW; ++mb)
 #pragma unroll
-    for (int nb = 0; nb < 2; ++nb) {
-      const int j = wn * 64 + nb * 32 + lr;
+    for (int nb = 0; nb < kW; ++nb) {
+      const int j = wn * SW + nb * 32 + lr;
       const float cn = s_cnorm[j];
       const float cs = s_cinv[j];
       const int ci = s_cimg[j];
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
-        const int i = wm * 64 + mb * 32 + (v >> 2) * 8 + lh * 4 + (v & 3);
+        const int i = wm * SW + mb * 32 + (v >> 2) * 8 + lh * 4 + (v & 3);
         const float d2 = fmaf(cs * s_rinv[i], acc[mb][nb][v], s_rnorm[i] + cn);  // clamped by min_key
         const int ri = s_rimg[i];
         E[i * EPITCH + j] = (ri == ci || ri == n || ci == n) ? __int_as_float(kInfBits) : d2;
@@ -487,7 +510,7 @@ __global__ __launch_bounds__(THREADS, kSplit ? 3 : 2) void msm_pair_min_kernel(
       }
       if (seg < n && cur != __int_as_float(kInfBits)) atomicMin(dst + seg, min_key(cur));
     }
-  } else {
+  } else if (t < BM + BN) {
     // Column pass: the same tile seen from the reference side (symmetric reuse).
     const int j = t - BM;
     const int cc = col0 + j;
@@ -511,27 +534,43 @@ __global__ __launch_bounds__(THREADS, kSplit ? 3 : 2) void msm_pair_min_kernel(
 }
 
 // Stage 2: the fp32 MFMA pairwise-minima kernel (leaves squared minima bits).
-int run_pairs(const float* z, int n, int p, int c, const Workspace& w, const Pools& pools, hipStream_t s) {
+template <int kW>
+int launch_pairs(const float* z, int n, int p, int c, const Workspace& w, const Pools& pools, hipStream_t s) {
+  constexpr int BM = tile_of(kW);
   const long long rows = (long long)n * p;
   const long long T = (rows + BM - 1) / BM;
   const long long ntiles = total_tiles(T);
   const long long grid = (ntiles + kXcds - 1) / kXcds * kXcds;
   if (grid > 0x7fffffffLL) return MUSC_ERR_UNSUPPORTED;
-#define MUSC_PAIR_LAUNCH(V4, SPLIT)                                                                              \
-  hipLaunchKernelGGL((msm_pair_min_kernel<V4, SPLIT>), dim3((unsigned)grid, pools.count), dim3(THREADS), 0, s, z,    \
+#define MUSC_PAIR_LAUNCH(V4, SPLIT)                                                                                \
+  hipLaunchKernelGGL((msm_pair_min_kernel<V4, SPLIT, kW>), dim3((unsigned)grid, pools.count), dim3(THREADS), 0, s, z, \
                      w.norms, w.inv, w.minbits, (int)rows, n, p, c, (int)T, ntiles, pools.ws_step)
-  const bool split = p >= BM;
-  // whole-chunk loads: c a multiple of two chunks, and a 128-row panel addressable with
+  // whole-chunk loads: c a multiple of two chunks, and a tile's panel addressable with
   // 32-bit offsets (any pool size: the buffer resources are based at each tile's panels)
-  if (c % (2 * BK) == 0 && (unsigned long long)BM * (unsigned long long)c * 4ull < (1ull << 31)) {
-    if (split) MUSC_PAIR_LAUNCH(2, true); else MUSC_PAIR_LAUNCH(2, false);
-  } else if ((c & 3) == 0) {
-    if (split) MUSC_PAIR_LAUNCH(1, true); else MUSC_PAIR_LAUNCH(1, false);
-  } else {
-    if (split) MUSC_PAIR_LAUNCH(0, true); else MUSC_PAIR_LAUNCH(0, false);
+  const bool chunks = c % (2 * BK) == 0 && (unsigned long long)BM * (unsigned long long)c * 4ull < (1ull << 31);
+  if (p >= BM) {
+    if (chunks) MUSC_PAIR_LAUNCH(2, true); else if ((c & 3) == 0) MUSC_PAIR_LAUNCH(1, true); else MUSC_PAIR_LAUNCH(0, true);
+  } else if constexpr (kW == 1) {
+    if (chunks) MUSC_PAIR_LAUNCH(2, false); else if ((c & 3) == 0) MUSC_PAIR_LAUNCH(1, false); else MUSC_PAIR_LAUNCH(0, false);
   }
 #undef MUSC_PAIR_LAUNCH
   return check_launch();
+}
+
+// 128-tiles need fewer operand bytes and LDS reads per MFMA, but three of them share a CU,
+// so a launch of a few thousand ends with most of its last round idle, and one below 768
+// leaves CUs empty throughout; 64-tiles are a quarter of that.  Measured by 128-tiles in the
+// launch (us, 64 against 128): 45 9.1 / 21.7, 120 21.4 / 37.8, 528 94 / 138, 820 180 / 237,
+// 1128 266 / 297, 3741 847 / 861, 5778 1277 / 1324, 7626 1751 / 1742, 8385 1404 / 1414, 11325
+// 2589 / 2545, 13861 2437 / 2363, 17020 2019 / 1971.  Patches per image below 128 always
+// take 64-tiles: a 128-tile could hold several image boundaries and reduced through LDS
+// (12403 tiles of P = 100: 2259 / 2534; P = 40, 3.96e4: 7548 / 8060).  Both tiles add a
+// dot product's terms in the same order: the same bits.
+constexpr long long kSmallTiles = 6000;
+int run_pairs(const float* z, int n, int p, int c, const Workspace& w, const Pools& pools, hipStream_t s) {
+  const long long T = ((long long)n * p + tile_of(2) - 1) / tile_of(2);
+  return p < tile_of(2) || total_tiles(T) * pools.count < kSmallTiles ? launch_pairs<1>(z, n, p, c, w, pools, s)
+                                                                      : launch_pairs<2>(z, n, p, c, w, pools, s);
 }
 
 }  // namespace msm

@@ -5,7 +5,7 @@ import torch
 
 import oracle
 from oracle import msm as om
-from musc_hip import _MSM_hip
+from musc_hip import _MSM_hip, pipeline
 from musc_hip import synthetic
 
 pytestmark = pytest.mark.gpu
@@ -195,3 +195,25 @@ def test_rank_selection_across_register_sizes(device, n):
         ref = om.MSM(z, lo, hi).numpy()
         err = np.abs(got - ref).max()
         assert err <= ATOL, (n, lo, hi, err)
+
+
+@pytest.mark.parametrize('n,p,c', [(4, 130, 33), (5, 128, 36), (3, 257, 64), (3, 301, 100), (7, 143, 32), (2, 1000, 4)])
+def test_both_tiles_of_the_pair_kernel_agree(device, n, p, c):
+    # one pool of these sizes takes 64-tiles; enough pools in one launch take 128-tiles, whose
+    # epilogues then meet image boundaries, padding and duplicated rows at every offset.  Both add
+    # the terms of a dot product in the same order: the same bits
+    tiles = -(-n * p // 128)
+    pools = 6000 // (tiles * (tiles + 1) // 2) + 1
+    g = torch.Generator(device='cuda').manual_seed(n * p + c)
+    z = torch.randn((1, pools, n, p, c), generator=g, device=device)
+    z[0, 1, 1, :7] = z[0, 1, 0, 5:12]
+    z[0, 2, 0, 3, 0] = float('nan')
+    before, pipeline.POOLS_WORKSPACE = pipeline.POOLS_WORKSPACE, 8 << 30
+    try:
+        for normalize in (True, False):
+            many = pipeline.msm_all(z, topmin_max=1, normalize_rows=normalize)
+            for k in list(range(0, pools, max(1, pools // 8))) + [1, 2]:
+                one = pipeline.msm_all(z[:, k:k + 1], topmin_max=1, normalize_rows=normalize)
+                assert torch.equal(many[0, k].view(torch.int64), one[0, 0].view(torch.int64)), k
+    finally:
+        pipeline.POOLS_WORKSPACE = before
