@@ -295,10 +295,11 @@ int musc_rscin_f32(const float* cls_tokens, const double* image_scores, int n, i
  *         the reference's evaluation transform run on the CPU
  *         (models/backbone/open_clip/transform.py:118-133, Pillow==11.1.0);
  * mean3, std3  host arrays of 3 floats (OPENAI_DATASET_MEAN / _STD for CLIP).
- * Workspace: musc_preprocess_workspace_bytes (coefficient tables, plus the uint8 output
- * of the horizontal pass when both axes are resampled and the band of source rows does
- * not fit the fused kernel's LDS, or in_w % 4 != 0).  When the fused kernel runs,
- * images must be 4-byte aligned (MUSC_ERR_INVALID_ARG otherwise).  Reduction factors up
+ * Workspace: musc_preprocess_workspace_bytes (coefficient tables, plus room for the uint8
+ * output of the horizontal pass unless both axes are resampled, in_w % 4 == 0, out_w <=
+ * 768 and neither axis has more than 15 taps; in that case images must be 4-byte aligned,
+ * MUSC_ERR_INVALID_ARG otherwise).  The room is used beyond 31 taps (reductions of more
+ * than 7.5) and where only the width is resampled.  Reduction factors up
  * to 15.5 per axis (64 taps); MUSC_ERR_UNSUPPORTED beyond, or for batch, in_h or out_h
  * above 65535. */
 int musc_preprocess_workspace_bytes(int batch, int in_h, int in_w, int out_h, int out_w, size_t* out);

@@ -68,37 +68,42 @@ __host__ __device__ inline int2 window(const AxisGeom& g, int in_size, int xx, d
   return make_int2(xmin, xmax - xmin);
 }
 
-// One thread per output index: bounds (xmin - shift, count) and a row of `width`
-// fixed-point coefficients (zero past the window).  identity: the axis keeps its size and is not resampled (window
-// {xx, 1}, coefficient 1.0, which reproduces the byte exactly).
-__global__ __launch_bounds__(kThreads) void coeff_kernel(int in_size, int out_size, int width, int shift,
-                                                         int identity, int2* __restrict__ bounds,
-                                                         int* __restrict__ kk) {
+// One axis of the coefficient launch.  identity: the axis keeps its size and is not
+// resampled (window {xx, 1}, coefficient 1.0, which reproduces the byte exactly).
+struct AxisTable {
+  AxisGeom g;
+  int in_size, out_size, shift, identity;
+  int2* bounds;
+  int* kk;
+};
+
+// Both axes' tables in one launch (3.3 us at 1024 -> 518), kLanes lanes per output index: bounds (xmin - shift,
+// count) and a row of `width` <= kLanes fixed-point coefficients (zero past the window).
+// Bound by latency: a lane forms one bicubic value and one quotient where a thread per
+// output index formed all of them one after the other.  The sum over the window stays in
+// Pillow's order (each lane adds the group's values in turn), so its rounding does too.
+template <int kLanes>
+__global__ __launch_bounds__(kThreads) void coeff_kernel(AxisTable h, AxisTable v, int width) {
 #pragma clang fp contract(off)
-  const int xx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (xx >= out_size) return;
-  int* k = kk + (long long)xx * width;
-  if (identity) {
-    bounds[xx] = make_int2(xx - shift, 1);
-    k[0] = 1 << kPrecisionBits;
-    for (int x = 1; x < width; ++x) k[x] = 0;
-    return;
+  const int unit = (blockIdx.x * kThreads + threadIdx.x) / kLanes, x = threadIdx.x % kLanes;
+  if (unit >= h.out_size + v.out_size) return;
+  const bool second = unit >= h.out_size;
+  const int xx = second ? unit - h.out_size : unit;
+  const AxisTable t = second ? v : h;
+  int2 w = make_int2(xx, 1);
+  int q = x == 0 ? 1 << kPrecisionBits : 0;
+  if (!t.identity) {
+    double center;
+    w = window(t.g, t.in_size, xx, &center);
+    double k = x < w.y ? bicubic((x + w.x - center + 0.5) * t.g.ss) : 0.0;
+    double ww = 0.0;
+    for (int i = 0; i < w.y; ++i) ww += __shfl(k, i, kLanes);
+    if (ww != 0.0) k /= ww;
+    q = k < 0 ? (int)(-0.5 + k * (1 << kPrecisionBits)) : (int)(0.5 + k * (1 << kPrecisionBits));
+    if (x >= w.y) q = 0;
   }
-  const AxisGeom g = axis_geom(in_size, out_size);
-  double center;
-  const int2 w = window(g, in_size, xx, &center);
-  double ww = 0.0;
-  for (int x = 0; x < w.y; ++x) ww += bicubic((x + w.x - center + 0.5) * g.ss);
-  for (int x = 0; x < width; ++x) {
-    int q = 0;
-    if (x < w.y) {
-      double v = bicubic((x + w.x - center + 0.5) * g.ss);
-      if (ww != 0.0) v /= ww;
-      q = v < 0 ? (int)(-0.5 + v * (1 << kPrecisionBits)) : (int)(0.5 + v * (1 << kPrecisionBits));
-    }
-    k[x] = q;
-  }
-  bounds[xx] = make_int2(w.x - shift, w.y);
+  if (x < width) t.kk[(long long)xx * width + x] = q;
+  if (x == 0) t.bounds[xx] = make_int2(w.x - t.shift, w.y);
 }
 
 __device__ inline int clip8(int acc) {
@@ -187,36 +192,28 @@ __global__ __launch_bounds__(kThreads) void vpass_kernel(const uint8_t* __restri
   store_normalised(out + (long long)b * 3 * plane + (long long)yy * w + xx, plane, s, nrm);
 }
 
-// Fused resize: one workgroup per (image, band of `band` output rows).  The source
-// rows the band's vertical windows cover stream through a double-buffered LDS row
-// (coalesced 4-byte loads, one row ahead in registers, one barrier per row), each is
-// resampled horizontally into an LDS block of uint8 rows, and the vertical pass +
-// ToTensor + Normalize then reads that block and writes the float32 planes.  The
-// uint8 intermediate never reaches HBM.  A thread owns output columns tid + 256 j
-// (j < kCols) in every row, so its horizontal coefficients are loaded into registers
-// once; the band's vertical coefficient rows sit in LDS.  kT is the larger of the
-// two axes' tap counts (odd, <= 15), kW its coefficient row width.  Needs
-// in_w % 4 == 0 (4-byte aligned rows) and out_w <= 256 * kCols; the host sizes
-// `band` and the dynamic LDS (fused_plan).
-constexpr int kRowRegs = 16;     // 4-byte words per thread per staged row (in_w * 3 <= 16 KB)
-constexpr int kCols = 3;         // output columns per thread (out_w <= 768)
-constexpr int kFusedMaxTaps = 15;
+// Fused resize: one workgroup per (image, band of output rows, up to 64 output columns).
+// The source rectangle under the tile's windows goes into LDS as aligned 4-byte words, all
+// its loads in flight at once; a wave then resamples one source row at a time (a lane owns
+// one output column and keeps its coefficients in registers) into an LDS block of one word
+// (R | G << 8 | B << 16) per pixel, and the vertical pass walks the output rows of the tile
+// the same way (coefficients uniform in the wave).  (u / 255 - mean) / std has 256 values
+// per channel: a table in LDS, formed with the same two divisions.  Two barriers in all,
+// and the uint8 intermediate never reaches HBM.  Any in_w and image alignment: a row's
+// words start at its address rounded down to 4, the remainder joins the window's offset.
+// Bound by instruction issue (a byte extraction and a 24-bit multiply-add per tap and
+// channel) and, below four images, by the launches.  Whole call, 1024 x 1024 -> 518: one
+// image 48.9 -> 18.4 us, 4 52.1 -> 20.9, 16 97.2 -> 52.5 against a band of 8 whole rows per
+// workgroup, its source rows staged one at a time with a barrier each; 4 of 1023 x 1023, whose
+// width took two passes through HBM, 57.1 -> 21.0.
+constexpr int kTileCols = kWave;      // output columns per tile at most: one per lane
+constexpr int kTileMaxBand = 16;
+constexpr int kTileMaxTaps = 31;
+constexpr int kWaves = kThreads / kWave;
+constexpr int kLoadRows = 4, kLoadWords = 2;  // rows x words of 64 lanes a wave loads at once
 
-struct FusedLayout {
-  int rowpad;        // bytes per staged source row (x2 buffers), with slack for the widest window read
-  int bstride;       // bytes per row of the uint8 block (out_w * 3 + 12 rounded up to 16)
-  int blk;           // bytes of the uint8 block (nrows x bstride)
-  size_t total;      // dynamic LDS bytes
-};
-
-__host__ __device__ inline FusedLayout fused_layout(int in_w, int out_w, int nrows, int band, int width) {
-  FusedLayout f;
-  f.rowpad = (in_w * 3 + 3 * width + 8 + 15) & ~15;
-  f.bstride = (out_w * 3 + 12 + 15) & ~15;      // the last 4-column group's 12 bytes stay in the row
-  f.blk = nrows * f.bstride;
-  f.total = 2 * (size_t)f.rowpad + f.blk + (size_t)band * width * 4 + (size_t)band * 8;
-  return f;
-}
+// 24-bit products: bytes times coefficients below 2 in 22-bit fixed point
+__device__ inline int mad24(uint32_t byte, int coeff, int acc) { return __mul24((int)byte, coeff) + acc; }
 
 // Horizontal tap sums of one output pixel from an LDS row: the window's 3*kT bytes
 // (kT = the axis' tap count, <= kW) start at byte a; they are read as aligned 4-byte
@@ -238,143 +235,147 @@ __device__ inline int3 hsum_words(const uint8_t* __restrict__ row, int a, const 
 #pragma unroll
   for (int x = 0; x < kT; ++x) {
     const int j = 3 * x;
-    s0 += (int)((e[j >> 2] >> (8 * (j & 3))) & 0xffu) * c[x];
-    s1 += (int)((e[(j + 1) >> 2] >> (8 * ((j + 1) & 3))) & 0xffu) * c[x];
-    s2 += (int)((e[(j + 2) >> 2] >> (8 * ((j + 2) & 3))) & 0xffu) * c[x];
+    s0 = mad24((e[j >> 2] >> (8 * (j & 3))) & 0xffu, c[x], s0);
+    s1 = mad24((e[(j + 1) >> 2] >> (8 * ((j + 1) & 3))) & 0xffu, c[x], s1);
+    s2 = mad24((e[(j + 2) >> 2] >> (8 * ((j + 2) & 3))) & 0xffu, c[x], s2);
   }
   return make_int3(s0, s1, s2);
 }
 
-template <int kW, int kT>
-__global__ __launch_bounds__(kThreads) void fused_kernel(const uint8_t* __restrict__ src, int in_h, int in_w,
-                                                         int out_h, int out_w, int band, int max_rows,
-                                                         const int2* __restrict__ bh, const int* __restrict__ kh,
-                                                         const int2* __restrict__ bv, const int* __restrict__ kv,
-                                                         Norm nrm, float* __restrict__ out) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  const int b = blockIdx.y, tid = threadIdx.x;
-  const int y0 = blockIdx.x * band;
-  const int y1 = min(y0 + band, out_h);
-  const int r0 = bv[y0].x;
-  const int nrows = bv[y1 - 1].x + bv[y1 - 1].y - r0;
-  // the host sized the LDS for max_rows source rows with the same window arithmetic
-  if (nrows > max_rows) return;
-  const FusedLayout f = fused_layout(in_w, out_w, max_rows, band, kW);
-  const int words = in_w * 3 / 4;                 // 4-byte words per source row
-  uint8_t* rowbuf = smem;                         // [2][rowpad]
-  uint8_t* blk = smem + 2 * f.rowpad;             // [nrows][out_w][3]
-  int* vk = reinterpret_cast<int*>(blk + f.blk);  // [band][kW] vertical coefficients of this band
-  int2* vb = reinterpret_cast<int2*>(vk + band * kW);
-  for (int i = tid; i < (y1 - y0) * kW; i += kThreads) vk[i] = kv[(long long)y0 * kW + i];
-  for (int i = tid; i < y1 - y0; i += kThreads) vb[i] = bv[y0 + i];
+// The word at p, which lies on a 4-byte boundary and may stick out of [first, end) at the
+// first or last bytes of the batch: bytes outside are not read.
+__device__ inline uint32_t image_word(const uint8_t* p, const uint8_t* first, const uint8_t* end) {
+  if (p >= first && p + 4 <= end) return *reinterpret_cast<const uint32_t*>(p);
+  uint32_t v = 0;
+  for (int i = 0; i < 4; ++i)
+    if (p + i >= first && p + i < end) v |= (uint32_t)p[i] << (8 * i);
+  return v;
+}
 
-  int2 hb[kCols];
-  int hc[kCols][kW];
+template <int kW, int kT>
+__global__ __launch_bounds__(kThreads) void tile_kernel(const uint8_t* __restrict__ src, int batch, int in_h,
+                                                        int in_w, int out_h, int out_w, int band, int cols,
+                                                        int max_rows, int pitch, const int2* __restrict__ bh,
+                                                        const int* __restrict__ kh, const int2* __restrict__ bv,
+                                                        const int* __restrict__ kv, Norm nrm,
+                                                        float* __restrict__ out) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];  // [max_rows][pitch] bytes | [max_rows][64] words
+  __shared__ float lut[3][256];
+  const int tid = threadIdx.x, lane = tid % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int x0 = blockIdx.x * cols, x1 = min(x0 + cols, out_w);
+  const int y0 = blockIdx.y * band, y1 = min(y0 + band, out_h);
+  const int r0 = bv[y0].x, nrows = bv[y1 - 1].x + bv[y1 - 1].y - r0;
+  const int c0 = bh[x0].x, c1 = bh[x1 - 1].x + bh[x1 - 1].y;
+  // the host sized the LDS with the same window arithmetic
+  if (nrows > max_rows || 3 * (c1 - c0) + 3 * kT + 16 > pitch) return;
+  uint32_t* const blk = reinterpret_cast<uint32_t*>(smem + max_rows * pitch);
+
+  const long long row_bytes = (long long)in_w * 3;
+  const uint8_t* const end = src + (long long)batch * in_h * row_bytes;
+  const uint8_t* const first = src + ((long long)blockIdx.z * in_h + r0) * row_bytes + 3 * c0;
+  const int mis0 = (int)(reinterpret_cast<uintptr_t>(first) & 3), row_mis = (int)(row_bytes & 3);
+  for (int r = wave; r < nrows; r += kWaves * kLoadRows) {
+    // row r + kWaves i: its words from the boundary below its first byte
+    for (int w0 = lane; 4 * w0 < 3 * (c1 - c0) + 3; w0 += kWave * kLoadWords) {
+      uint32_t v[kLoadRows][kLoadWords];
 #pragma unroll
-  for (int j = 0; j < kCols; ++j) {
-    const int xx = tid + j * kThreads;
-    hb[j] = make_int2(0, 0);
-    if (xx < out_w) {
-      hb[j] = bh[xx];
-      load_coeffs<kW>(kh + (long long)xx * kW, hc[j]);
-    } else {
+      for (int i = 0; i < kLoadRows; ++i) {
+        const int rr = r + i * kWaves, mis = (mis0 + rr * row_mis) & 3;
+        const int words = rr < nrows ? (mis + 3 * (c1 - c0) + 3) / 4 : 0;
+        const uint8_t* p = first + rr * row_bytes - mis;
 #pragma unroll
-      for (int x = 0; x < kW; ++x) hc[j][x] = 0;
+        for (int j = 0; j < kLoadWords; ++j) {
+          const int w = w0 + j * kWave;
+          v[i][j] = w < words ? image_word(p + 4 * w, src, end) : 0u;
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < kLoadRows; ++i)
+#pragma unroll
+        for (int j = 0; j < kLoadWords; ++j) {
+          const int rr = r + i * kWaves, w = w0 + j * kWave;
+          if (rr < nrows && 4 * w < pitch) *reinterpret_cast<uint32_t*>(smem + rr * pitch + 4 * w) = v[i][j];
+        }
     }
   }
+  const bool active = x0 + lane < x1;
+  const int xx = active ? x0 + lane : x1 - 1;
+  int hc[kW];
+  load_coeffs<kW>(kh + (long long)xx * kW, hc);
+  const int off = 3 * (bh[xx].x - c0);
+#pragma unroll
+  for (int c = 0; c < 3; ++c) lut[c][tid] = ((float)tid / 255.0f - nrm.mean[c]) / nrm.stdv[c];
+  __syncthreads();
 
-  const uint32_t* img = reinterpret_cast<const uint32_t*>(src + (long long)b * in_h * in_w * 3);
-  uint32_t stage[kRowRegs];
-  auto load_row = [&](int r) {
-    const uint32_t* g = img + (long long)(r0 + r) * words;
-#pragma unroll
-    for (int i = 0; i < kRowRegs; ++i) {
-      const int w = tid + i * kThreads;
-      if (w < words) stage[i] = g[w];
-    }
-  };
-  load_row(0);
-  for (int r = 0; r < nrows; ++r) {
-    uint32_t* buf = reinterpret_cast<uint32_t*>(rowbuf + (r & 1) * f.rowpad);
-#pragma unroll
-    for (int i = 0; i < kRowRegs; ++i) {
-      const int w = tid + i * kThreads;
-      if (w < words) buf[w] = stage[i];
-    }
-    if (r + 1 < nrows) load_row(r + 1);
-    __syncthreads();
-    const uint8_t* row = rowbuf + (r & 1) * f.rowpad;
-    uint8_t* dst = blk + r * f.bstride;
-#pragma unroll
-    for (int j = 0; j < kCols; ++j) {
-      const int xx = tid + j * kThreads;
-      if (xx < out_w) {
-        // taps past the window carry weight 0; they read the row's slack bytes
-        const int3 s = hsum_words<kW, kT>(row, hb[j].x * 3, hc[j]);
-        dst[xx * 3 + 0] = (uint8_t)clip8(s.x);
-        dst[xx * 3 + 1] = (uint8_t)clip8(s.y);
-        dst[xx * 3 + 2] = (uint8_t)clip8(s.z);
-      }
-    }
+  for (int r = wave; r < nrows; r += kWaves) {
+    // taps past the window carry weight 0; they read the row's slack bytes
+    const int3 s = hsum_words<kW, kT>(smem + r * pitch, off + ((mis0 + r * row_mis) & 3), hc);
+    blk[r * kWave + lane] = clip8(s.x) | clip8(s.y) << 8 | clip8(s.z) << 16;
   }
   __syncthreads();
-  // vertical pass: a thread takes 4 adjacent output columns (12 bytes = 3 aligned words
-  // of a block row per tap; the padded row stride keeps them aligned)
+
   const long long plane = (long long)out_h * out_w;
-  float* o = out + (long long)b * 3 * plane;
-  const int groups = (out_w + 3) / 4;
-  const int n = (y1 - y0) * groups;
-  for (int idx = tid; idx < n; idx += kThreads) {
-    const int yl = idx / groups, x0 = 4 * (idx % groups);
-    const int2 bd = vb[yl];
-    int c[kW];
+  float* o = out + (long long)blockIdx.z * 3 * plane + x0 + lane;
+  for (int y = y0 + wave; y < y1; y += kWaves) {
+    const int top = bv[y].x - r0;
+    int s0 = 1 << (kPrecisionBits - 1), s1 = s0, s2 = s0;
 #pragma unroll
-    for (int x = 0; x < kW; ++x) c[x] = vk[yl * kW + x];
-    int acc[12];
-#pragma unroll
-    for (int q = 0; q < 12; ++q) acc[q] = 1 << (kPrecisionBits - 1);
-#pragma unroll
-    for (int y = 0; y < kT; ++y) {
-      const int rr = min(bd.x - r0 + y, nrows - 1);     // weight 0 past the window
-      const uint32_t* w = reinterpret_cast<const uint32_t*>(blk + rr * f.bstride + x0 * 3);
-      const uint32_t d[3] = {w[0], w[1], w[2]};
-#pragma unroll
-      for (int q = 0; q < 12; ++q) acc[q] += (int)((d[q >> 2] >> (8 * (q & 3))) & 0xffu) * c[y];
+    for (int t = 0; t < kT; ++t) {
+      const int c = kv[(long long)y * kW + t];
+      const uint32_t u = blk[min(top + t, nrows - 1) * kWave + lane];  // weight 0 past the window
+      s0 = mad24(u & 0xffu, c, s0);
+      s1 = mad24((u >> 8) & 0xffu, c, s1);
+      s2 = mad24((u >> 16) & 0xffu, c, s2);
     }
-    float* orow = o + (long long)(y0 + yl) * out_w + x0;
-#pragma unroll
-    for (int px = 0; px < 4; ++px) {
-      if (x0 + px < out_w)
-        store_normalised(orow + px, plane, make_int3(acc[3 * px], acc[3 * px + 1], acc[3 * px + 2]), nrm);
+    if (active) {
+      o[(long long)y * out_w] = lut[0][clip8(s0)];
+      o[(long long)y * out_w + plane] = lut[1][clip8(s1)];
+      o[(long long)y * out_w + 2 * plane] = lut[2][clip8(s2)];
     }
   }
 }
 
-// Band (output rows per workgroup) and LDS of the fused kernel, or band 0 when it does
-// not apply: the largest band (<= 32 rows) whose block fits 64 KB.  Larger bands
-// recompute fewer halo rows, smaller blocks let more workgroups share a CU; measured at
-// 1024 -> 518 the 64 KB choice (band 8, three workgroups per CU) beat both a 40 KB one
-// (band 4) and a 78 KB one (band 16, two per CU; 14 % slower).
-constexpr size_t kFusedLdsBudget = 64 * 1024;
+// Tile of the fused kernel, or band 0 when it does not apply (more than 31 taps; there the
+// passes through HBM read each source row once, a tile several times).  Up to 31 taps the
+// tile is ahead throughout: 1400 x 1365 -> 224 (27 taps, 3 images) 69.5 -> 38.2 us, 1000 x
+// 777 -> 224 (6 images) 75.9 -> 26.5, 300 x 300 -> 224 (1) 55.0 -> 17.6.  Columns:
+// equal tiles of at most 64.  Band: the more output rows share a source row, the fewer
+// source rows are resampled twice, but the rectangle must leave room for several
+// workgroups per CU, and the grid must fill the chip.
+constexpr size_t kTileLds = 32 * 1024, kTileLdsMax = 60 * 1024;
+constexpr long long kTileGrid = 1024;
 
-struct FusedPlan {
-  int band, max_rows;
+struct TilePlan {
+  int band, cols, max_rows, pitch;
   size_t lds;
 };
 
-inline FusedPlan fused_plan(int in_h, int in_w, int out_h, int out_w, const AxisGeom& gv, int taps, int width) {
-  FusedPlan best{0, 0, 0};
-  if (in_w % 4 != 0 || in_w * 3 > kRowRegs * kThreads * 4 || out_w > kCols * kThreads || taps > kFusedMaxTaps)
-    return best;
-  for (int band = 32; band >= 1; band /= 2) {
+inline TilePlan tile_plan(int batch, int in_h, int in_w, int out_h, int out_w, const AxisGeom& gh, const AxisGeom& gv,
+                          int taps) {
+  TilePlan best{0, 0, 0, 0, 0};
+  if (taps > kTileMaxTaps) return best;
+  const int tiles = (out_w + kTileCols - 1) / kTileCols;
+  best.cols = ((out_w + tiles - 1) / tiles + 3) & ~3;
+  auto extent = [](const AxisGeom& g, int in_size, int out_size, int step) {  // most source rows or columns of a tile
     int worst = 0;
-    for (int y0 = 0; y0 < out_h; y0 += band) {
-      const int y1 = y0 + band < out_h ? y0 + band : out_h;
-      const int2 a = window(gv, in_h, y0, nullptr), z = window(gv, in_h, y1 - 1, nullptr);
+    for (int i = 0; i < out_size; i += step) {
+      const int j = i + step < out_size ? i + step : out_size;
+      const int2 a = window(g, in_size, i, nullptr), z = window(g, in_size, j - 1, nullptr);
       worst = worst > z.x + z.y - a.x ? worst : z.x + z.y - a.x;
     }
-    const FusedLayout f = fused_layout(in_w, out_w, worst, band, width);
-    if (f.total <= kFusedLdsBudget) return FusedPlan{band, worst, f.total};
+    return worst;
+  };
+  // a row: its words, and what the widest instantiated window reads past them
+  best.pitch = (3 * extent(gh, in_w, out_w, best.cols) + 3 * kTileMaxTaps + 16 + 3) & ~3;
+  for (int band = kTileMaxBand; band >= 1; band /= 2) {
+    best.max_rows = extent(gv, in_h, out_h, band);
+    best.lds = (size_t)best.max_rows * (best.pitch + 4 * kWave);
+    const long long grid = (long long)batch * tiles * ((out_h + band - 1) / band);
+    if (band > 4 ? best.lds <= kTileLds && grid >= kTileGrid : best.lds <= kTileLdsMax) {
+      best.band = band;
+      return best;
+    }
   }
   return best;
 }
@@ -391,9 +392,8 @@ inline int table_width(int taps) {
 struct Plan {
   AxisGeom gh, gv;
   bool need_h, need_v;
-  int band;                  // > 0: the fused kernel runs with this many output rows per workgroup
-  int max_rows;              // fused kernel: most source rows a band reads
-  size_t lds;                // fused kernel: dynamic LDS bytes
+  TilePlan tile;             // fused kernel, when tile.band > 0
+  bool words;                // images must be 4-byte aligned, and no uint8 intermediate is reserved
   int width;                 // coefficient row width (both axes): a bucket >= the taps of either axis
   int taps;                  // the larger of the two axes' tap counts
   int row0, rows;            // source rows the vertical pass reads (horizontal pass extent)
@@ -410,11 +410,10 @@ inline Plan plan(int batch, int in_h, int in_w, int out_h, int out_w) {
   if (!p.need_v) p.gv.taps = 1;
   p.taps = p.gh.taps > p.gv.taps ? p.gh.taps : p.gv.taps;
   p.width = table_width(p.taps);
-  const FusedPlan fp = (p.need_h && p.need_v) ? fused_plan(in_h, in_w, out_h, out_w, p.gv, p.taps, p.width)
-                                              : FusedPlan{0, 0, 0};
-  p.band = fp.band;
-  p.max_rows = fp.max_rows;
-  p.lds = fp.lds;
+  const bool both = p.need_h && p.need_v;
+  p.tile = both ? tile_plan(batch, in_h, in_w, out_h, out_w, p.gh, p.gv, p.taps) : TilePlan{0, 0, 0, 0, 0};
+  // what the interface states; the fused kernel itself takes other widths and alignments too
+  p.words = both && in_w % 4 == 0 && out_w <= 768 && p.taps <= 15;
   if (p.need_h && p.need_v) {
     const int2 first = window(p.gv, in_h, 0, nullptr);
     const int2 last = window(p.gv, in_h, out_h - 1, nullptr);
@@ -434,7 +433,7 @@ inline Plan plan(int batch, int in_h, int in_w, int out_h, int out_w) {
   p.off_kv = off;
   off = align_up(off + (size_t)out_h * p.width * sizeof(int), 256);
   p.off_tmp = off;
-  if (p.need_h && p.band == 0) off = align_up(off + (size_t)batch * p.rows * out_w * 3, 256);
+  if (p.need_h && !p.words) off = align_up(off + (size_t)batch * p.rows * out_w * 3, 256);
   p.total = off;
   return p;
 }
@@ -468,7 +467,7 @@ extern "C" int musc_preprocess_u8(const uint8_t* images, int batch, int in_h, in
   int rc = prep::validate(batch, in_h, in_w, out_h, out_w);
   if (rc) return rc;
   const prep::Plan p = prep::plan(batch, in_h, in_w, out_h, out_w);
-  if (p.band > 0 && (reinterpret_cast<uintptr_t>(images) & 3) != 0) return MUSC_ERR_INVALID_ARG;
+  if (p.words && (reinterpret_cast<uintptr_t>(images) & 3) != 0) return MUSC_ERR_INVALID_ARG;
   if (!workspace || workspace_bytes < p.total) return MUSC_ERR_WORKSPACE;
   prep::Norm nrm;
   for (int c = 0; c < 3; ++c) {
@@ -484,25 +483,41 @@ extern "C" int musc_preprocess_u8(const uint8_t* images, int batch, int in_h, in
   auto* tmp = reinterpret_cast<uint8_t*>(ws + p.off_tmp);
   const int T = prep::kThreads;
   // the two-pass path reads the horizontal pass's rows from 0; the fused kernel reads source rows
-  const int vshift = (p.need_h && p.band == 0) ? p.row0 : 0;
-  hipLaunchKernelGGL(prep::coeff_kernel, dim3((out_w + T - 1) / T), dim3(T), 0, stream, in_w, out_w, p.width, 0,
-                     p.need_h ? 0 : 1, bh, kh);
-  hipLaunchKernelGGL(prep::coeff_kernel, dim3((out_h + T - 1) / T), dim3(T), 0, stream, in_h, out_h, p.width,
-                     vshift, p.need_v ? 0 : 1, bv, kv);
-  if (p.band > 0) {
-#define MUSC_PREP_FUSED(W, TAPS)                                                                                   \
-  hipLaunchKernelGGL((prep::fused_kernel<W, TAPS>), dim3((out_h + p.band - 1) / p.band, batch), dim3(T), p.lds,    \
-                     stream, images, in_h, in_w, out_h, out_w, p.band, p.max_rows, bh, kh, bv, kv, nrm, out)
-    switch (p.taps) {
-      case 1: case 3: case 5: MUSC_PREP_FUSED(8, 5); break;   // taps are odd; short windows use 5 (zero weights)
-      case 7: MUSC_PREP_FUSED(8, 7); break;
-      case 9: MUSC_PREP_FUSED(12, 9); break;
-      case 11: MUSC_PREP_FUSED(12, 11); break;
-      case 13: MUSC_PREP_FUSED(16, 13); break;
-      case 15: MUSC_PREP_FUSED(16, 15); break;
+  const int vshift = (p.need_h && p.tile.band == 0) ? p.row0 : 0;
+  const prep::AxisTable th{p.gh, in_w, out_w, 0, p.need_h ? 0 : 1, bh, kh};
+  const prep::AxisTable tv{p.gv, in_h, out_h, vshift, p.need_v ? 0 : 1, bv, kv};
+#define MUSC_PREP_COEFF(L)                                                                                         \
+  hipLaunchKernelGGL(prep::coeff_kernel<L>, dim3((unsigned)(((long long)(out_w + out_h) * L + T - 1) / T)), dim3(T), \
+                     0, stream, th, tv, p.width)
+  if (p.width <= 16) {
+    MUSC_PREP_COEFF(16);
+  } else if (p.width <= 32) {
+    MUSC_PREP_COEFF(32);
+  } else {
+    MUSC_PREP_COEFF(64);
+  }
+#undef MUSC_PREP_COEFF
+  const prep::TilePlan& tp = p.tile;
+  if (tp.band > 0) {
+#define MUSC_PREP_TILE(W, TAPS)                                                                                    \
+  hipLaunchKernelGGL((prep::tile_kernel<W, TAPS>),                                                                 \
+                     dim3((out_w + tp.cols - 1) / tp.cols, (out_h + tp.band - 1) / tp.band, batch), dim3(T), tp.lds, \
+                     stream, images, batch, in_h, in_w, out_h, out_w, tp.band, tp.cols, tp.max_rows, tp.pitch, bh,  \
+                     kh, bv, kv, nrm, out)
+    switch (p.taps) {  // odd, at least 5 when an axis is resampled
+      case 5: MUSC_PREP_TILE(8, 5); break;
+      case 7: MUSC_PREP_TILE(8, 7); break;
+      case 9: MUSC_PREP_TILE(12, 9); break;
+      case 11: MUSC_PREP_TILE(12, 11); break;
+      case 13: MUSC_PREP_TILE(16, 13); break;
+      case 15: MUSC_PREP_TILE(16, 15); break;
+      case 17: case 19: MUSC_PREP_TILE(24, 19); break;
+      case 21: case 23: MUSC_PREP_TILE(24, 23); break;
+      case 25: case 27: MUSC_PREP_TILE(32, 27); break;
+      case 29: case 31: MUSC_PREP_TILE(32, 31); break;
       default: return MUSC_ERR_UNSUPPORTED;
     }
-#undef MUSC_PREP_FUSED
+#undef MUSC_PREP_TILE
     return check_launch();
   }
 #define MUSC_PREP_LAUNCH(W)                                                                                        \

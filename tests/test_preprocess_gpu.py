@@ -44,6 +44,22 @@ def test_matches_the_cpu_transform_bit_for_bit(device, src, size):
     assert torch.equal(got, ref)
 
 
+# the fused kernel's edges: one output column, one full tile of 64 columns and one more,
+# tiles of unequal width, bands of 16 to 1 output rows with a remainder, rows at every byte
+# alignment (in_w % 4 = 1, 2, 3) up to the last bytes of the batch, the tap counts past 15
+# (17, 23, 25, 31) and the first that goes through two passes (33)
+@pytest.mark.parametrize('src,size', [((40, 7), (9, 1)), ((61, 129), (17, 64)), ((61, 130), (33, 65)),
+                                      ((200, 131), (130, 190)), ((401, 403), (101, 102)), ((543, 335), (100, 67)),
+                                      ((602, 301), (100, 67)), ((749, 101), (100, 131)), ((801, 99), (100, 70)),
+                                      ((1024, 1021), (518, 518))])
+@pytest.mark.parametrize('b', [1, 3])
+def test_tile_edges_bit_for_bit(device, src, size, b):
+    imgs = _images(b, *src, seed=src[0] + src[1])
+    got = _preprocess.preprocess_u8(torch.from_numpy(imgs).to(device), size).cpu()
+    ref = torch.stack([op.to_tensor_normalize(op.resize_bicubic_u8(im, *size)) for im in imgs], 0)
+    assert torch.equal(got, ref)
+
+
 def test_resized_bytes_equal_pillow(device):
     from PIL import Image
     imgs = _images(2, 640, 480, 7)
