@@ -15,6 +15,8 @@
 // hence the integer passes, identical.  ToTensor (u8 / 255) and Normalize ((x -
 // mean) / std) are fused into the vertical pass as correctly rounded float32
 // division and subtraction, the operations torch performs on the CPU.
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace musc {
@@ -202,15 +204,17 @@ __global__ __launch_bounds__(kThreads) void vpass_kernel(const uint8_t* __restri
 // and the uint8 intermediate never reaches HBM.  Any in_w and image alignment: a row's
 // words start at its address rounded down to 4, the remainder joins the window's offset.
 // Bound by instruction issue (a byte extraction and a 24-bit multiply-add per tap and
-// channel) and, below four images, by the launches.  Whole call, 1024 x 1024 -> 518: one
-// image 48.9 -> 18.4 us, 4 52.1 -> 20.9, 16 97.2 -> 52.5 against a band of 8 whole rows per
+// channel) and, up to four images, by the host and the launches.  Whole call, 1024 x 1024 ->
+// 518: one image 48.9 -> 18.2 us, 4 51.9 -> 18.6, 16 97.1 -> 42.9 against a band of 8 whole rows per
 // workgroup, its source rows staged one at a time with a barrier each; 4 of 1023 x 1023, whose
-// width took two passes through HBM, 57.1 -> 21.0.
+// width took two passes through HBM, 56.9 -> 18.6.  With a test of every word
+// against the batch's ends, which put each load behind its own branch and wait, 16 images took
+// 52.5 us; tiles away from the ends now go without.
 constexpr int kTileCols = kWave;      // output columns per tile at most: one per lane
 constexpr int kTileMaxBand = 16;
 constexpr int kTileMaxTaps = 31;
 constexpr int kWaves = kThreads / kWave;
-constexpr int kLoadRows = 4, kLoadWords = 2;  // rows x words of 64 lanes a wave loads at once
+constexpr int kLoadRows = 5, kLoadWords = 2;  // rows x words of 64 lanes a wave loads at once
 
 // 24-bit products: bytes times coefficients below 2 in 22-bit fixed point
 __device__ inline int mad24(uint32_t byte, int coeff, int acc) { return __mul24((int)byte, coeff) + acc; }
@@ -275,29 +279,50 @@ __global__ __launch_bounds__(kThreads) void tile_kernel(const uint8_t* __restric
   const uint8_t* const end = src + (long long)batch * in_h * row_bytes;
   const uint8_t* const first = src + ((long long)blockIdx.z * in_h + r0) * row_bytes + 3 * c0;
   const int mis0 = (int)(reinterpret_cast<uintptr_t>(first) & 3), row_mis = (int)(row_bytes & 3);
-  for (int r = wave; r < nrows; r += kWaves * kLoadRows) {
-    // row r + kWaves i: its words from the boundary below its first byte
-    for (int w0 = lane; 4 * w0 < 3 * (c1 - c0) + 3; w0 += kWave * kLoadWords) {
-      uint32_t v[kLoadRows][kLoadWords];
+  const int seg = 3 * (c1 - c0);  // bytes of a row
+  auto row_word = [&](int rr) {   // the boundary below the row's first byte
+    return first + rr * row_bytes - ((mis0 + rr * row_mis) & 3);
+  };
+  auto stage = [&](auto whole) {
+    for (int r = wave; r < nrows; r += kWaves * kLoadRows) {
+      for (int w0 = 0; 4 * w0 < seg + 3; w0 += kWave * kLoadWords) {
+        uint32_t v[kLoadRows][kLoadWords];
 #pragma unroll
-      for (int i = 0; i < kLoadRows; ++i) {
-        const int rr = r + i * kWaves, mis = (mis0 + rr * row_mis) & 3;
-        const int words = rr < nrows ? (mis + 3 * (c1 - c0) + 3) / 4 : 0;
-        const uint8_t* p = first + rr * row_bytes - mis;
+        for (int i = 0; i < kLoadRows; ++i) {
+          // past the rectangle its last row and word are loaded again, never stored
+          const int rr = min(r + i * kWaves, nrows - 1);
+          const int last = (((mis0 + rr * row_mis) & 3) + seg - 1) / 4;
+          const uint8_t* p = row_word(rr);
 #pragma unroll
-        for (int j = 0; j < kLoadWords; ++j) {
-          const int w = w0 + j * kWave;
-          v[i][j] = w < words ? image_word(p + 4 * w, src, end) : 0u;
+          for (int j = 0; j < kLoadWords; ++j) {
+            const uint32_t at = 4 * (uint32_t)min(w0 + j * kWave + lane, last);
+            if constexpr (decltype(whole)::value) {
+              v[i][j] = *reinterpret_cast<const uint32_t*>(p + at);
+            } else {
+              v[i][j] = image_word(p + at, src, end);
+            }
+          }
         }
+        // every load before the first wait (the compiler sinks one into its store's branch)
+#pragma unroll
+        for (int i = 0; i < kLoadRows; ++i)
+#pragma unroll
+          for (int j = 0; j < kLoadWords; ++j) asm volatile("" : "+v"(v[i][j]));
+#pragma unroll
+        for (int i = 0; i < kLoadRows; ++i)
+#pragma unroll
+          for (int j = 0; j < kLoadWords; ++j) {
+            const int rr = r + i * kWaves, w = w0 + j * kWave + lane;
+            if (rr < nrows && 4 * w < seg + 3) *reinterpret_cast<uint32_t*>(smem + rr * pitch + 4 * w) = v[i][j];
+          }
       }
-#pragma unroll
-      for (int i = 0; i < kLoadRows; ++i)
-#pragma unroll
-        for (int j = 0; j < kLoadWords; ++j) {
-          const int rr = r + i * kWaves, w = w0 + j * kWave;
-          if (rr < nrows && 4 * w < pitch) *reinterpret_cast<uint32_t*>(smem + rr * pitch + 4 * w) = v[i][j];
-        }
     }
+  };
+  // a rectangle whose words all lie inside the batch needs no test per word
+  if (row_word(0) >= src && row_word(nrows - 1) + seg + 6 <= end) {
+    stage(std::true_type{});
+  } else {
+    stage(std::false_type{});
   }
   const bool active = x0 + lane < x1;
   const int xx = active ? x0 + lane : x1 - 1;
@@ -338,8 +363,8 @@ __global__ __launch_bounds__(kThreads) void tile_kernel(const uint8_t* __restric
 
 // Tile of the fused kernel, or band 0 when it does not apply (more than 31 taps; there the
 // passes through HBM read each source row once, a tile several times).  Up to 31 taps the
-// tile is ahead throughout: 1400 x 1365 -> 224 (27 taps, 3 images) 69.5 -> 38.2 us, 1000 x
-// 777 -> 224 (6 images) 75.9 -> 26.5, 300 x 300 -> 224 (1) 55.0 -> 17.6.  Columns:
+// tile is ahead throughout: 1400 x 1365 -> 224 (27 taps, 3 images) 69.4 -> 34.5 us, 1000 x
+// 777 -> 224 (6 images) 75.8 -> 23.3, 300 x 300 -> 224 (1) 55.1 -> 17.9.  Columns:
 // equal tiles of at most 64.  Band: the more output rows share a source row, the fewer
 // source rows are resampled twice, but the rectangle must leave room for several
 // workgroups per CU, and the grid must fill the chip.
