@@ -8,7 +8,10 @@
 //
 // MI355X design
 //   lnamd_stats_kernel     per (image, layer): kChunks workgroups stream disjoint
-//                          slices and write shifted fp64 partial sums.
+//                          slices and write shifted fp64 partial sums, eight loads in
+//                          flight per thread (16 images, 4 fp16 layers: one load at a
+//                          time left the pass at 59 us = 3.0 TB/s; the call over three
+//                          radii 429 -> 405 us).
 //   lnamd_finalize_kernel  per (image, layer): mean and 1/sqrt(var + eps).
 //   lnamd_stream_kernel    default path.  One workgroup per (image, layer, slice of
 //                          4*cg channels); thread (column, 4 channels) sweeps the
@@ -16,7 +19,10 @@
 //                          column in a register ring, puts the nested vertical sums
 //                          of each output row in LDS (double-buffered, one barrier
 //                          per row) and adds its horizontal neighbours'.  Every
-//                          token is read once, every output written once.
+//                          token is read once, every output written once.  Where the
+//                          columns alone do not fill the chip (a few images), they are
+//                          split into bands of rows: a whole column is 37 dependent
+//                          rows long whatever the batch.
 //   lnamd_pool_kernel      L2-normalising path.  One workgroup per (image, layer, output row); each
 //                          thread owns 4 channels.  It sweeps the row's columns,
 //                          reading the 2*hmax+1 input rows once per column, keeps
@@ -37,6 +43,7 @@ namespace lnamd {
 constexpr int kChunks = 16;       // stats workgroups per (image, layer)
 constexpr int kMaxRadii = 4;
 constexpr int kMaxHalo = 4;       // radius <= 9
+constexpr int kStreamGrid = 512;  // streaming workgroups below which rows are split into bands
 constexpr int kColBatch = 4;      // columns per normalisation barrier
 
 struct Radii {
@@ -101,12 +108,21 @@ __global__ __launch_bounds__(256) void lnamd_stats_kernel(TokenPtrs tokens, int 
   const long long per = (n4 + kChunks - 1) / kChunks;
   const long long lo = chunk * per, hi = lo + per < n4 ? lo + per : n4;
   double s = 0.0, ss = 0.0;
-  for (long long i = lo + threadIdx.x; i < hi; i += blockDim.x) {
-    const float4 v = load4_once<kDtype>(base, first / 4 + i);
+  auto add = [&](float4 v) {
     const float d0 = v.x - shift, d1 = v.y - shift, d2 = v.z - shift, d3 = v.w - shift;
     s += (double)d0 + (double)d1 + (double)d2 + (double)d3;
     ss += (double)d0 * d0 + (double)d1 * d1 + (double)d2 * d2 + (double)d3 * d3;
+  };
+  constexpr int kAhead = 8;  // loads in flight per thread
+  long long i = lo + threadIdx.x;
+  for (; i + (kAhead - 1) * (long long)blockDim.x < hi; i += kAhead * (long long)blockDim.x) {
+    float4 v[kAhead];
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) v[j] = load4_once<kDtype>(base, first / 4 + i + j * (long long)blockDim.x);
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) add(v[j]);
   }
+  for (; i < hi; i += blockDim.x) add(load4_once<kDtype>(base, first / 4 + i));
   s = wave_sum(s);
   ss = wave_sum(ss);
   __shared__ double red[2][4];
@@ -339,14 +355,17 @@ template <int kDtype, int kHalo, int kNR, bool kPool>
 __global__ __launch_bounds__(1024) void lnamd_stream_kernel(TokenPtrs tokens, int n_layers, int batch,
                                                             int tokens_per_image, int c, int has_cls, int side,
                                                             int cg, int slices, Radii radii, Radii slot, int raw,
-                                                            int layout, int pool, const double* __restrict__ stats,
+                                                            int layout, int pool, int band,
+                                                            const double* __restrict__ stats,
                                                             float* __restrict__ out) {
   extern __shared__ float4 vsum[];  // [2][kNR][side * cg], then (kPool) hsum [kNR][side * cg]
   // XCD-grouped order: the slices of one (image, layer) run on one XCD (-3 % time
   // at config 2, measured).  The grid is padded to a multiple of kXcds.
   const long long wid = xcd_logical_id(blockIdx.x, gridDim.x);
-  if (wid >= (long long)batch * n_layers * slices) return;
-  const int unit = (int)(wid / slices), slice = (int)(wid % slices);
+  const int bands = (side + band - 1) / band;
+  if (wid >= (long long)batch * n_layers * slices * bands) return;
+  const int slice = (int)(wid % slices), unit = (int)(wid / slices / bands);
+  const int h0 = (int)(wid / slices % bands) * band, h1 = min(h0 + band, side);  // this workgroup's output rows
   const int b = unit / n_layers, l = unit % n_layers;
   const int w = threadIdx.x / cg, gl = threadIdx.x % cg;
   const int groups = c / 4;
@@ -370,19 +389,20 @@ __global__ __launch_bounds__(1024) void lnamd_stream_kernel(TokenPtrs tokens, in
   float4 ring[2 * kHalo + 1];
 #pragma unroll
   for (int i = 0; i < 2 * kHalo + 1; ++i) ring[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-  float4 next = load4_once<kDtype>(base, col_base4);
+  const int first = max(h0 - kHalo, 0), end = min(h1 + kHalo, side);  // source rows
+  float4 next = load4_once<kDtype>(base, col_base4 + (long long)first * row_step4);
 
-  for (int hi = 0; hi < side + kHalo; ++hi) {
+  for (int hi = first; hi < h1 + kHalo; ++hi) {
     float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (hi < side) {
+    if (hi < end) {
       x = make_float4(next.x - mean, next.y - mean, next.z - mean, next.w - mean);
-      if (hi + 1 < side) next = load4_once<kDtype>(base, col_base4 + (long long)(hi + 1) * row_step4);
+      if (hi + 1 < end) next = load4_once<kDtype>(base, col_base4 + (long long)(hi + 1) * row_step4);
     }
 #pragma unroll
     for (int i = 0; i < 2 * kHalo; ++i) ring[i] = ring[i + 1];
     ring[2 * kHalo] = x;
     const int h = hi - kHalo;
-    if (h < 0) continue;
+    if (h < h0) continue;
     // nested vertical sums of row h (ring index kHalo) for the ascending radii
     float4* buf = vsum + (size_t)(h & 1) * kNR * row_len;
     {
@@ -483,11 +503,11 @@ __global__ __launch_bounds__(1024) void lnamd_stream_kernel(TokenPtrs tokens, in
 template <int kDtype, int kHalo, bool kPool>
 int dispatch_stream_nr(int nr, dim3 grid, dim3 block, size_t smem, hipStream_t s, const TokenPtrs& tp, int n_layers,
                        int batch, int tpi, int c, int has_cls, int side, int cg, int slices, const Radii& radii,
-                       const Radii& slot, int raw, int layout, int pool, const double* stats, float* out) {
+                       const Radii& slot, int raw, int layout, int pool, int band, const double* stats, float* out) {
 #define MUSC_STREAM_CASE(NR)                                                                                      \
   case NR:                                                                                                        \
     hipLaunchKernelGGL((lnamd_stream_kernel<kDtype, kHalo, NR, kPool>), grid, block, smem, s, tp, n_layers, batch, \
-                       tpi, c, has_cls, side, cg, slices, radii, slot, raw, layout, pool, stats, out);            \
+                       tpi, c, has_cls, side, cg, slices, radii, slot, raw, layout, pool, band, stats, out);      \
     break;
   switch (nr) {
     MUSC_STREAM_CASE(1)
@@ -503,12 +523,12 @@ int dispatch_stream_nr(int nr, dim3 grid, dim3 block, size_t smem, hipStream_t s
 template <int kDtype, bool kPool>
 int dispatch_stream(int halo, int nr, dim3 grid, dim3 block, size_t smem, hipStream_t s, const TokenPtrs& tp,
                     int n_layers, int batch, int tpi, int c, int has_cls, int side, int cg, int slices,
-                    const Radii& radii, const Radii& slot, int raw, int layout, int pool, const double* stats,
+                    const Radii& radii, const Radii& slot, int raw, int layout, int pool, int band, const double* stats,
                     float* out) {
 #define MUSC_STREAM_HALO(H)                                                                                      \
   case H:                                                                                                        \
     return dispatch_stream_nr<kDtype, H, kPool>(nr, grid, block, smem, s, tp, n_layers, batch, tpi, c, has_cls,   \
-                                                side, cg, slices, radii, slot, raw, layout, pool, stats, out);
+                                                side, cg, slices, radii, slot, raw, layout, pool, band, stats, out);
   switch (halo) {
     MUSC_STREAM_HALO(0)
     MUSC_STREAM_HALO(1)
@@ -700,22 +720,34 @@ int lnamd_run(const void* const* tokens, int n_layers, int in_dtype, int batch, 
     const int slices = (groups + cg - 1) / cg;
     const int threads = side * cg;
     const int raw = (flags & MUSC_LNAMD_RAW_SUMS) ? 1 : 0;
-    const dim3 grid((unsigned)((units * slices + kXcds - 1) / kXcds * kXcds));
+    // Rows per workgroup: the whole column where the grid fills the chip; a few images are
+    // split into bands, which read their 2 * halo neighbouring rows again (from L2) but
+    // sweep fewer rows one after the other.  Pooling sums across rows and is not split.
+    // Whole call with and without bands (37 x 37 x 1024 fp32): 3 images, r = 1, 24.6 against
+    // 72.8 us; 8 images 36.2 / 81.0; 8 images, r = 1, 3, 5, 58.9 / 112.5; 16 images 94.0 /
+    // 133.7 (the statistics pass' share included).
+    int band = side;
+    const int least = halo < 1 ? 4 : 4 * halo;
+    if (!pooled)
+      while (band > least && (long long)units * slices * ((side + band - 1) / band) < kStreamGrid)
+        band = band / 2 > least ? (band + 1) / 2 : least;
+    const long long work = (long long)units * slices * ((side + band - 1) / band);
+    const dim3 grid((unsigned)((work + kXcds - 1) / kXcds * kXcds));
     const int pool = pooled ? pool_side : side;
     if (in_dtype == MUSC_DTYPE_F32)
       rc = pooled ? dispatch_stream<MUSC_DTYPE_F32, true>(halo, n_radii, grid, dim3(threads), smem, stream, tp,
                                                          n_layers, batch, tokens_per_image, c, has_cls, side, cg,
-                                                         slices, rr, slot, raw, out_layout, pool, stats, out)
+                                                         slices, rr, slot, raw, out_layout, pool, band, stats, out)
                   : dispatch_stream<MUSC_DTYPE_F32, false>(halo, n_radii, grid, dim3(threads), smem, stream, tp,
                                                           n_layers, batch, tokens_per_image, c, has_cls, side, cg,
-                                                          slices, rr, slot, raw, out_layout, pool, stats, out);
+                                                          slices, rr, slot, raw, out_layout, pool, band, stats, out);
     else
       rc = pooled ? dispatch_stream<MUSC_DTYPE_F16, true>(halo, n_radii, grid, dim3(threads), smem, stream, tp,
                                                          n_layers, batch, tokens_per_image, c, has_cls, side, cg,
-                                                         slices, rr, slot, raw, out_layout, pool, stats, out)
+                                                         slices, rr, slot, raw, out_layout, pool, band, stats, out)
                   : dispatch_stream<MUSC_DTYPE_F16, false>(halo, n_radii, grid, dim3(threads), smem, stream, tp,
                                                           n_layers, batch, tokens_per_image, c, has_cls, side, cg,
-                                                          slices, rr, slot, raw, out_layout, pool, stats, out);
+                                                          slices, rr, slot, raw, out_layout, pool, band, stats, out);
   }
   if (rc) return rc;
   return check_launch();

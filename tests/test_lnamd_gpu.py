@@ -59,6 +59,24 @@ def test_wide_radii_in_any_order(device, side, c):
         assert err <= ATOL, f'r={r} (L2): {err}'
 
 
+@pytest.mark.parametrize('side,radii', [(1, [1]), (4, [1]), (5, [1]), (9, [3, 1]), (8, [5]), (17, [1, 3, 5]),
+                                        (37, [3]), (33, [9, 1, 7])])
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float16])
+def test_row_bands_equal_whole_columns(device, side, radii, dtype):
+    # one image alone is split into bands of rows (down to 4, or 4 halos), 520 images (one
+    # 64-channel slice each) are not: the same sums in the same order
+    g = torch.Generator().manual_seed(side)
+    few = (torch.randn((2, side * side + 1, 64), generator=g) + 0.5).to(dtype).to(device)
+    many = few.repeat(260, 1, 1)
+    for raw in (False, True):
+        whole = _lnamd_hip.lnamd([many], radii, raw_sums=raw)
+        split = _lnamd_hip.lnamd([few], radii, raw_sums=raw)
+        assert torch.equal(split, whole[:, :2]) and torch.equal(split, whole[:, -2:])
+    for k, r in enumerate(radii):
+        ref = ol.aggregate_direct([few.float().cpu()], r)
+        assert (_lnamd_hip.lnamd([few], radii)[k].cpu() - ref).abs().max().item() <= ATOL
+
+
 def test_fused_l2norm(device):
     g = torch.Generator().manual_seed(5)
     feats = [torch.randn((4, 1370, 1024), generator=g) for _ in range(3)]
