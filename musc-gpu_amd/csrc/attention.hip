@@ -323,13 +323,19 @@ __device__ inline uint32_t abs_max4(const float (&x)[4]) {
   return max(max(abs_bits(x[0]), abs_bits(x[1])), max(abs_bits(x[2]), abs_bits(x[3])));
 }
 // (a, b) -> hi = fp16 of each (one packed conversion, to nearest even), lo = fp16 of the exact
-// remainder x - hi (one mixed-precision fused multiply-add each, rounded once)
+// remainder x - hi, as one mixed-precision fused multiply-add each (v_fma_mixlo/mixhi_f16,
+// rounded once).  The -1 is hidden from the optimizer, which would turn the multiply-adds into
+// separate conversions and subtractions.  The instructions are the compiler's own: those of an
+// asm statement are not counted when it keeps the two wait states a matrix instruction needs
+// after the vector instruction that wrote its operand.
 typedef float float2v __attribute__((ext_vector_type(2)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 __device__ inline void split2(float a, float b, half2v& hi, half2v& lo) {
   hi = __builtin_convertvector((float2v{a, b}), half2v);
-  asm("v_fma_mixlo_f16 %0, %1, -1.0, %2 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "=v"(lo) : "v"(hi), "v"(a));
-  asm("v_fma_mixhi_f16 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(lo) : "v"(hi), "v"(b));
+  float minus_one = -1.f;
+  asm("" : "+s"(minus_one));
+  lo[0] = (_Float16)__builtin_fmaf((float)hi[0], minus_one, a);
+  lo[1] = (_Float16)__builtin_fmaf((float)hi[1], minus_one, b);
 }
 
 __global__ __launch_bounds__(WAVES32 * kWave, 1) void attn_fwd_kernel(const float* __restrict__ qg,
