@@ -289,8 +289,8 @@ constexpr int VR16 = D + 8;        // V block pitch (halves), row-major: 144 B r
 //      limit): 22 bits, or within 2^-32 of the largest probability for smaller ones.
 // A tile whose inputs the split does not represent to 22 bits (an entry past fp16's range
 // after scaling, 16 neighbouring entries of a row all below 2^-3 but not zero, a
-// non-finite entry, a scale out of range) is noticed while it is staged and computed
-// again by attend_tile_f32, so such inputs cost time, never accuracy.
+// non-finite entry, a scale out of range, a logit of 2^20 and more in log2 units) is
+// noticed and computed again by attend_tile_f32, so such inputs cost time, never accuracy.
 //   Layout: one 12-wave workgroup (384 queries, three waves per SIMD) per CU: the barrier
 // keeps the waves in step, where of three 4-wave workgroups on a CU the oldest finishes
 // first and the last runs alone.  Waves 0-7 stage: one float4 of K and one of V per
@@ -311,6 +311,10 @@ constexpr int kSplitSmem = 2 * kGroup * 4 * kPlane * 2;
 constexpr int kF32KernelSmem = kSplitSmem > kF32Smem ? kSplitSmem : kF32Smem;
 constexpr float kPShift = 7.f;                 // probabilities are scaled by 2^7
 constexpr float kSplitMax = 60000.f;           // largest scaled entry (fp16 holds 65504)
+// largest block maximum in log2 units: base is rounded to 2^-4 or better below it, so a probability
+// stays under 2^15.1.  Beyond, base (a rounded product) and the probability's exponent (the product
+// unrounded, less base) part ways by whole units, past fp16's range.
+constexpr float kSplitLogit = 0x1p20f;
 constexpr float kSplitMin = 0.125f;            // smallest scaled 16-entry group maximum: lo is exact to 2^-25
 
 // 2^k with x 2^k in [2^9, 2^10) for the largest |x| (given by its bits); 1 for zero or denormal
@@ -517,6 +521,7 @@ __global__ __launch_bounds__(WAVES32 * kWave, 1) void attn_fwd_kernel(const floa
 #pragma unroll
     for (int v = 1; v < 16; ++v) bmax = __builtin_elementwise_maximum(bmax, s[v]);
     bmax = halves_max(bmax) * c;
+    bad = bad || !(fabsf(bmax) < kSplitLogit);
     // lazy rescaling: the running maximum moves only past kLazyLog2
     if (!__all(bmax <= base + (kPShift + kLazyLog2))) {
       const float bnew = fmaxf(base, bmax - kPShift);

@@ -185,3 +185,24 @@ def test_fp32_non_finite_entries(device, where, value):
         sure = ~torch.isfinite(ref[1])
         assert not torch.isfinite(out[1][sure]).any()
         torch.testing.assert_close(out[1][~sure], ref[1][~sure], rtol=1e-4, atol=2e-5)
+
+
+@pytest.mark.parametrize('a', [1e2, 1e3, 1e4, 3e4, 1e5, 1e6])
+def test_fp32_large_logits(device, a):
+    # logits of 1e4 to 1e12.  An fp32 logit is off by at most 2 x 64 x 2^-24 |q||k| scale; where the
+    # two largest are further apart than that (and than 20 for exp(-20)) the output is the value row
+    # of the largest, elsewhere it lies within the values' range
+    g = torch.Generator().manual_seed(11)
+    q, k = (torch.randn((2, 256, 64), generator=g) * a for _ in range(2))
+    v = torch.randn((2, 256, 64), generator=g)
+    out = _attention_hip.attention(q.to(device), k.to(device), v.to(device), 0.125).cpu().double()
+    assert torch.isfinite(out).all()
+    logits = torch.bmm(q.double() * 0.125, k.double().transpose(1, 2).contiguous())
+    top = logits.topk(2, dim=-1)
+    bound = 2.0 ** -17 * q.double().norm(dim=-1) * k.double().norm(dim=-1).max() * 0.125
+    sure = top.values[..., 0] - top.values[..., 1] > 2 * bound + 20
+    assert sure.float().mean() > (0.9 if a >= 1e3 else 0.5)
+    ref = torch.stack([v[b].double()[top.indices[b, :, 0]] for b in range(2)])
+    torch.testing.assert_close(out[sure], ref[sure], rtol=0, atol=1e-5)
+    assert (out <= v.double().amax(1, keepdim=True) + 1e-5).all()
+    assert (out >= v.double().amin(1, keepdim=True) - 1e-5).all()
