@@ -313,6 +313,10 @@ int musc_preprocess_u8(const uint8_t* images, int batch, int in_h, int in_w, int
 
 /* q, k, v, out  (bh, t, d) contiguous, dtype MUSC_DTYPE_F32 or MUSC_DTYPE_F16
  *               (fp16 storage, fp32 softmax and accumulation).
+ * fp32: products are three fp16 matrix products of operands held in 22 bits (Q by row and
+ * channel, K and V by channel), accumulated in fp32: a logit is off by a few 2^-22 of its
+ * sum of |q_c k_c| scale, an output by a few 2^-22 of its V channel's largest entry.  384-query
+ * tiles whose inputs do not fit that are computed with fp32 products.
  * Replaces the bmm -> softmax -> bmm of nn.MultiheadAttention inside
  * models/backbone/open_clip/transformer.py:232-234 and the fused softmax
  * models/modules/_attention_gpu.py:41-81,115-146.  d must be 64. */

@@ -282,15 +282,19 @@ constexpr int VR16 = D + 8;        // V block pitch (halves), row-major: 144 B r
 // restated for fp16 MFMA): three v_mfma_f32_32x32x16_f16 (32 cycles each) do what eight
 // v_mfma_f32_32x32x2f32 (64 cycles each) did.  The dropped lo.lo term and the rounding of lo
 // are below 2^-22 of the operands' size, the order of the fp32 sums' own rounding.
-//   Q  scaled per row (a lane owns a query), K and V by one power of two per head, taken
-//      from the head's first key block: its largest entry goes to [2^9, 2^10).  The
-//      logits' scale 2^-(..) is applied with the subtraction of the running maximum.
+//   K and V are scaled per channel, by the power of two that takes the channel's largest
+// entry among the head's first 32 keys to [2^9, 2^10), so a channel much smaller than its
+// neighbours keeps its 22 bits.  What K's scales differ by from the head's (at most 2^32)
+// is taken out of Q's channels, Q then scaled per row (a lane owns a query); the logits'
+// scale 2^-(..) is applied with the subtraction of the running maximum, V's when the
+// output is written.  A logit is off by a few 2^-22 of its sum of |q_c k_c| (q_c against
+// the row's, k_c against its channel's usual size), an output by 2^-22 of its channel's.
 //   P  formed as 2^(s - base) with base = running maximum - 7 (at most 2^15 at the lazy
 //      limit): 22 bits, or within 2^-32 of the largest probability for smaller ones.
-// A tile whose inputs the split does not represent to 22 bits (an entry past fp16's range
-// after scaling, 16 neighbouring entries of a row all below 2^-3 but not zero, a
-// non-finite entry, a scale out of range, a logit of 2^20 and more in log2 units) is
-// noticed and computed again by attend_tile_f32, so such inputs cost time, never accuracy.
+// A tile whose inputs the split does not represent so (an entry past fp16's range after
+// scaling, 16 neighbouring entries of a row all below 2^-3 but not zero, a non-finite
+// entry, a query row below 2^-90, a scale out of range, a logit of 2^20 and more in log2
+// units) is noticed and computed again by attend_tile_f32.
 //   Layout: one 12-wave workgroup (384 queries, three waves per SIMD) per CU: the barrier
 // keeps the waves in step, where of three 4-wave workgroups on a CU the oldest finishes
 // first and the last runs alone.  Waves 0-7 stage: one float4 of K and one of V per
@@ -317,10 +321,11 @@ constexpr float kSplitMax = 60000.f;           // largest scaled entry (fp16 hol
 constexpr float kSplitLogit = 0x1p20f;
 constexpr float kSplitMin = 0.125f;            // smallest scaled 16-entry group maximum: lo is exact to 2^-25
 
-// 2^k with x 2^k in [2^9, 2^10) for the largest |x| (given by its bits); 1 for zero or denormal
+// 2^k with x 2^k in [2^9, 2^10) for the largest |x| (given by its bits), or as near as a
+// normal 2^k comes; 1 for zero
 __device__ inline float split_scale(uint32_t max_bits) {
   const int e = (int)(max_bits >> 23);
-  return e == 0 ? 1.f : __uint_as_float((uint32_t)min(max(127 + 9 + 127 - e, 1), 254) << 23);
+  return max_bits == 0 ? 1.f : __uint_as_float((uint32_t)min(max(127 + 9 + 127 - e, 1), 254) << 23);
 }
 __device__ inline uint32_t abs_bits(float x) { return __float_as_uint(x) & 0x7fffffffu; }
 __device__ inline uint32_t abs_max4(const float (&x)[4]) {
@@ -348,7 +353,10 @@ __global__ __launch_bounds__(WAVES32 * kWave, 1) void attn_fwd_kernel(const floa
                                                                       float* __restrict__ og, int t, float scale_log2,
                                                                       HeadLayout in, HeadLayout out, int nbh) {
   __shared__ __attribute__((aligned(16))) unsigned char smem[kF32KernelSmem];
-  __shared__ uint32_t s_max[2][8];
+  __shared__ __attribute__((aligned(16))) uint32_t s_max[2][8][D];  // K, V: by wave and channel
+  // scales of K and V, what K's takes out of Q, 1 / V's
+  __shared__ __attribute__((aligned(16))) float s_kscale[D], s_vscale[D], s_qfold[D], s_vinv[D];
+  __shared__ float s_khead;
   _Float16* const planes = reinterpret_cast<_Float16*>(smem);
 
   const int2 unit = fwd_unit<QW * WAVES32>(t, nbh);
@@ -390,29 +398,80 @@ __global__ __launch_bounds__(WAVES32 * kWave, 1) void attn_fwd_kernel(const floa
     load_kv(0, x0);
     load_kv(1, x1);
   }
-  // this lane's query row: 8 m + lh halves of each 16-channel step, split, scaled by qscale
+  // this lane's query row: channels 16 m + 8 lh + (0..7) of the 16-channel steps m
+  float qx[4][8];
+#pragma unroll
+  for (int m = 0; m < 4; ++m)
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      const float4 v = q < t ? *reinterpret_cast<const float4*>(qg + head + (long long)q * st + 16 * m + 8 * lh + 4 * g)
+                             : make_float4(0.f, 0.f, 0.f, 0.f);
+      qx[m][4 * g] = v.x; qx[m][4 * g + 1] = v.y; qx[m][4 * g + 2] = v.z; qx[m][4 * g + 3] = v.w;
+    }
+  // the scales, from the head's first block: channel maxima of each staging wave's four keys,
+  // then wave 0 (K) and wave 1 (V) with a channel per lane
+  if (stager) {
+#pragma unroll
+    for (int op = 0; op < 2; ++op) {
+      uint32_t m[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        m[j] = abs_bits(op == 0 ? x0.k[j] : x0.v[j]);
+        m[j] = max(m[j], (uint32_t)__shfl_xor((int)m[j], 16, kWave));
+        m[j] = max(m[j], (uint32_t)__shfl_xor((int)m[j], 32, kWave));
+      }
+      if (lane < 16) *reinterpret_cast<uint4*>(&s_max[op][wave][sd4]) = make_uint4(m[0], m[1], m[2], m[3]);
+    }
+  }
+  __syncthreads();
+  if (wave < 2) {
+    uint32_t m = 0;
+#pragma unroll
+    for (int w = 0; w < 8; ++w) m = max(m, s_max[wave][w][lane]);
+    uint32_t all = m;
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) all = max(all, (uint32_t)__shfl_xor((int)all, off, kWave));
+    const float of_head = split_scale(all);
+    // a channel that is zero in the first block takes the head's scale
+    const float of_channel = m == 0 ? of_head : split_scale(m);
+    if (wave == 0) {
+      const float k = fminf(of_channel, of_head * 0x1p32f);
+      s_kscale[lane] = k;
+      s_qfold[lane] = of_head / k;  // powers of two: exact
+      if (lane == 0) s_khead = of_head;
+    } else {
+      s_vscale[lane] = of_channel;
+      s_vinv[lane] = 1.f / of_channel;
+    }
+  }
+  __syncthreads();
+  // the query split, scaled by qscale
   half8 qh[4], ql[4];
   float qscale;
   bool bad = false;  // this thread saw an entry the split does not represent
   {
-    float qx[4][8];
-    uint32_t qmax = 0;
+    uint32_t qraw = 0, qmax = 0;
 #pragma unroll
     for (int m = 0; m < 4; ++m)
 #pragma unroll
       for (int g = 0; g < 2; ++g) {
-        const float4 v = q < t ? *reinterpret_cast<const float4*>(qg + head + (long long)q * st + 16 * m + 8 * lh + 4 * g)
-                               : make_float4(0.f, 0.f, 0.f, 0.f);
-        qx[m][4 * g] = v.x; qx[m][4 * g + 1] = v.y; qx[m][4 * g + 2] = v.z; qx[m][4 * g + 3] = v.w;
-        const float q4[4] = {v.x, v.y, v.z, v.w};
+        const float4 f = *reinterpret_cast<const float4*>(&s_qfold[16 * m + 8 * lh + 4 * g]);
+        const float fold[4] = {f.x, f.y, f.z, f.w};
+        float q4[4] = {qx[m][4 * g], qx[m][4 * g + 1], qx[m][4 * g + 2], qx[m][4 * g + 3]};
+        qraw = max(qraw, abs_max4(q4));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) qx[m][4 * g + e] = q4[e] = q4[e] * fold[e];
         qmax = max(qmax, abs_max4(q4));
       }
     {
       const auto r = __builtin_amdgcn_permlane32_swap(qmax, qmax, false, false);
       qmax = max(r[0], r[1]);
+      const auto w = __builtin_amdgcn_permlane32_swap(qraw, qraw, false, false);
+      qraw = max(w[0], w[1]);
     }
     qscale = split_scale(qmax);
-    bad = qmax >= 0x7f800000u;
+    // a row so small that the folded entries could be denormal; NaN and inf
+    bad = qraw >= 0x7f800000u || (qraw < __float_as_uint(0x1p-90f) && qraw != 0);
     const float sgn = scale_log2 < 0.f ? -qscale : qscale;  // the logits' scale stays positive
 #pragma unroll
     for (int m = 0; m < 4; ++m)
@@ -423,30 +482,16 @@ __global__ __launch_bounds__(WAVES32 * kWave, 1) void attn_fwd_kernel(const floa
         ql[m][j] = (_Float16)(v - (float)qh[m][j]);
       }
   }
-  // the head's scales, from its first block
-  if (stager) {
-    uint32_t mk = abs_max4(x0.k), mv = abs_max4(x0.v);
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-      mk = max(mk, (uint32_t)__shfl_xor((int)mk, off, kWave));
-      mv = max(mv, (uint32_t)__shfl_xor((int)mv, off, kWave));
-    }
-    if (lane == 0) {
-      s_max[0][wave] = mk;
-      s_max[1][wave] = mv;
-    }
+  float kscale[4], vscale[4];  // of this thread's staged channels
+  {
+    const float4 k = *reinterpret_cast<const float4*>(&s_kscale[sd4]), v = *reinterpret_cast<const float4*>(&s_vscale[sd4]);
+    kscale[0] = k.x; kscale[1] = k.y; kscale[2] = k.z; kscale[3] = k.w;
+    vscale[0] = v.x; vscale[1] = v.y; vscale[2] = v.z; vscale[3] = v.w;
   }
-  __syncthreads();
-  uint32_t kmax = 0, vmax = 0;
-#pragma unroll
-  for (int w = 0; w < 8; ++w) {
-    kmax = max(kmax, s_max[0][w]);
-    vmax = max(vmax, s_max[1][w]);
-  }
-  const float kscale = split_scale(kmax), vscale = split_scale(vmax);
-  // c turns a product of scaled operands into log2 units; tiny scales (a zero softmax scale
-  // among them) are held at the smallest normal number, which moves no logit
-  const float c_raw = fabsf(scale_log2) / qscale / kscale;
+  // c turns a product of scaled operands into log2 units: |scale_log2| / (qscale khead), rounded
+  // once; tiny scales (a zero softmax scale among them) are held at the smallest normal number,
+  // which moves no logit
+  const float c_raw = ldexpf(fabsf(scale_log2), 254 - (int)(__float_as_uint(qscale) >> 23) - (int)(__float_as_uint(s_khead) >> 23));
   bad = bad || !(c_raw < 0x1p100f);
   const float c = fmaxf(c_raw, 0x1p-126f);
 
@@ -457,7 +502,7 @@ __global__ __launch_bounds__(WAVES32 * kWave, 1) void attn_fwd_kernel(const floa
     for (int op = 0; op < 2; ++op) {
       float x[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) x[j] = op == 0 ? in_regs.k[j] * kscale : in_regs.v[j] * vscale;
+      for (int j = 0; j < 4; ++j) x[j] = op == 0 ? in_regs.k[j] * kscale[j] : in_regs.v[j] * vscale[j];
       // largest of 16 neighbouring entries of the row (four lanes); NaN and inf order last
       int g = (int)abs_max4(x);
       g = max(g, __builtin_amdgcn_update_dpp(0, g, 0xb1, 0xf, 0xf, false));
@@ -583,12 +628,16 @@ __global__ __launch_bounds__(WAVES32 * kWave, 1) void attn_fwd_kernel(const floa
   }
   l = halves_sum(l);
   if (q < t) {
-    const float inv = 1.f / l / vscale;
+    const float inv = 1.f / l;  // and 1 / V's scale separately: their product may be denormal
     // register v of tile dt holds d = 32*dt + (v/4)*8 + 4h + v%4
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
-      const float4 a = make_float4(o0[4 * g] * inv, o0[4 * g + 1] * inv, o0[4 * g + 2] * inv, o0[4 * g + 3] * inv);
-      const float4 b = make_float4(o1[4 * g] * inv, o1[4 * g + 1] * inv, o1[4 * g + 2] * inv, o1[4 * g + 3] * inv);
+      const float4 va = *reinterpret_cast<const float4*>(&s_vinv[8 * g + 4 * lh]);
+      const float4 vb = *reinterpret_cast<const float4*>(&s_vinv[32 + 8 * g + 4 * lh]);
+      const float4 a = make_float4(o0[4 * g] * inv * va.x, o0[4 * g + 1] * inv * va.y, o0[4 * g + 2] * inv * va.z,
+                                   o0[4 * g + 3] * inv * va.w);
+      const float4 b = make_float4(o1[4 * g] * inv * vb.x, o1[4 * g + 1] * inv * vb.y, o1[4 * g + 2] * inv * vb.z,
+                                   o1[4 * g + 3] * inv * vb.w);
       float* orow = og + out.base(unit.x) + (long long)q * out.st;
       *reinterpret_cast<float4*>(orow + 8 * g + 4 * lh) = a;
       *reinterpret_cast<float4*>(orow + 32 + 8 * g + 4 * lh) = b;

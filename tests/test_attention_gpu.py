@@ -206,3 +206,55 @@ def test_fp32_large_logits(device, a):
     torch.testing.assert_close(out[sure], ref[sure], rtol=0, atol=1e-5)
     assert (out <= v.double().amax(1, keepdim=True) + 1e-5).all()
     assert (out >= v.double().amin(1, keepdim=True) - 1e-5).all()
+
+
+@pytest.mark.parametrize('factors', [((5, 1e-5), (20, 1e-6), (40, 1e-11)), ((41, 1e-20), (63, 1e4), (17, 1e12))])
+def test_fp32_channels_of_very_different_size_in_v(device, factors):
+    # an output column is a mean of its own V column, so its error is that column's: logits within
+    # 2^-20 of |q||k| scale (below 8 here), products within 2^-22 of the column's largest entry
+    g = torch.Generator().manual_seed(3)
+    q, k, v = (torch.randn((3, 300, 64), generator=g) for _ in range(3))
+    for c, f in factors:
+        v[:, :, c] *= f
+    v[1] *= 1e-20
+    out = _attention_hip.attention(q.to(device), k.to(device), v.to(device), 0.0625).cpu().double()
+    err = (out - _f64(q, k, v, 0.0625)).abs().amax(1)
+    assert (err <= 2.0 ** -17 * v.double().abs().amax(1)).all(), (err / v.double().abs().amax(1)).max()
+
+
+@pytest.mark.parametrize('fold', [1e6, 1e-6, 1e9])
+def test_fp32_channels_of_very_different_size_in_q_and_k(device, fold):
+    # channels large in q and as much smaller in k: each logit is still a sum of ordinary products,
+    # off by a few 2^-22 of the sum of |q_c k_c| scale (about 5, 2^-22 per split entry and fp32 sum),
+    # and an output by that times the spread of v (2-norm: the standard deviation)
+    g = torch.Generator().manual_seed(4)
+    q, k, v = (torch.randn((3, 300, 64), generator=g) for _ in range(3))
+    for c in (7, 8, 33):
+        q[:, :, c] *= fold
+        k[:, :, c] /= fold
+    out = _attention_hip.attention(q.to(device), k.to(device), v.to(device), 0.125).cpu().double()
+    ref = _f64(q, k, v, 0.125)
+    products = torch.bmm(q.double().abs(), k.double().abs().transpose(1, 2).contiguous()).mean() * 0.125
+    assert (out - ref).norm() / ref.norm() <= 2.0 ** -21 * products.item(), (out - ref).norm() / ref.norm()
+
+
+@pytest.mark.parametrize('size', [1e-33, 1e-35, 1e-37, 3e-39])
+def test_fp32_smallest_values(device, size):
+    # V down to denormal numbers: relative to the largest entry as any other V, but for the last
+    # place of a denormal result (2^-149) and of denormal entries
+    g = torch.Generator().manual_seed(6)
+    q, k, v = (torch.randn((2, 150, 64), generator=g) for _ in range(3))
+    v *= size
+    out = _attention_hip.attention(q.to(device), k.to(device), v.to(device), 0.125).cpu().double()
+    err = (out - _f64(q, k, v, 0.125)).abs().max().item()
+    assert err <= 2.0 ** -18 * v.abs().max().item() + 2.0 ** -148
+
+
+@pytest.mark.parametrize('q_size,k_size', [(1e-25, 1e25), (1e-36, 1e36), (1e25, 1e-25), (1e36, 1e-36), (1e-36, 1e-2)])
+def test_fp32_sizes_of_q_and_k_that_cancel(device, q_size, k_size):
+    g = torch.Generator().manual_seed(7)
+    q, k, v = (torch.randn((2, 150, 64), generator=g) for _ in range(3))
+    q, k = q * q_size, k * k_size
+    k[:, :, 9] *= 1e-3
+    out = _attention_hip.attention(q.to(device), k.to(device), v.to(device), 0.125).cpu().double()
+    torch.testing.assert_close(out, _f64(q, k, v, 0.125), rtol=0, atol=2.0 ** -18 * v.abs().max().item())
