@@ -294,7 +294,10 @@ constexpr int VR16 = D + 8;        // V block pitch (halves), row-major: 144 B r
 // A tile whose inputs the split does not represent so (an entry past fp16's range after
 // scaling, 16 neighbouring entries of a row all below 2^-3 but not zero, a non-finite
 // entry, a query row below 2^-90, a scale out of range, a logit of 2^20 and more in log2
-// units) is noticed and computed again by attend_tile_f32.
+// units) is noticed and computed again by attend_tile_f32: the split loop is left after the
+// group of blocks that follows the one in which it was seen.  Cost of every tile taking that
+// way, at the shape below: 275 us when seen in the first blocks or in Q, 307 us half way, 349 us
+// in the last block, against 267 us of the fp32 MFMA tiles alone.
 //   Layout: one 12-wave workgroup (384 queries, three waves per SIMD) per CU: the barrier
 // keeps the waves in step, where of three 4-wave workgroups on a CU the oldest finishes
 // first and the last runs alone.  Waves 0-7 stage: one float4 of K and one of V per
@@ -357,6 +360,7 @@ __global__ __launch_bounds__(WAVES32 * kWave, 1) void attn_fwd_kernel(const floa
   // scales of K and V, what K's takes out of Q, 1 / V's
   __shared__ __attribute__((aligned(16))) float s_kscale[D], s_vscale[D], s_qfold[D], s_vinv[D];
   __shared__ float s_khead;
+  __shared__ uint32_t s_bad[2];  // by parity of the group in which a thread first saw a bad entry
   _Float16* const planes = reinterpret_cast<_Float16*>(smem);
 
   const int2 unit = fwd_unit<QW * WAVES32>(t, nbh);
@@ -423,6 +427,7 @@ __global__ __launch_bounds__(WAVES32 * kWave, 1) void attn_fwd_kernel(const floa
       if (lane < 16) *reinterpret_cast<uint4*>(&s_max[op][wave][sd4]) = make_uint4(m[0], m[1], m[2], m[3]);
     }
   }
+  if (threadIdx.x < 2) s_bad[threadIdx.x] = 0;
   __syncthreads();
   if (wave < 2) {
     uint32_t m = 0;
@@ -532,11 +537,11 @@ __global__ __launch_bounds__(WAVES32 * kWave, 1) void attn_fwd_kernel(const floa
       load_kv(kb + 3, x1);
     }
   }
+  if (bad) s_bad[1] = 1;
   // V^T fragments through the transposing read, as in the fp16 kernel below
   const int vrd = (4 * lh + ((lq & 15) >> 2)) * SP32 + 16 * (lq >> 4) + 4 * (lq & 3);
   auto step = [&](int kb, Staged& x) {
     const _Float16* buf = planes + (kb & (2 * kGroup - 1)) * 4 * kPlane;
-    if ((kb & (kGroup - 1)) == 0) __syncthreads();
     floatx16 s;
     if (active) {
 #pragma unroll
@@ -616,9 +621,19 @@ __global__ __launch_bounds__(WAVES32 * kWave, 1) void attn_fwd_kernel(const floa
       o1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[0][1], ph[mm], o1, 0, 0, 0);
     }
   };
-  for (int kb = 0; kb < nkb; kb += 2) {
+  // Group g of kGroup blocks, from one barrier to the next, reads what was marked in group
+  // g - 1, complete before its barrier, and marks the other word; g + 1 marks this one again
+  // only after the next barrier, past which no wave of group g has its read before it.  So
+  // every wave leaves after the same group.
+  static_assert(kGroup == 2, "a turn of the loop is a group");
+  for (int kb = 0; kb < nkb; kb += kGroup) {
+    __syncthreads();
+    const int group = kb / kGroup;
+    const uint32_t marked = s_bad[(group + 1) & 1];
     step(kb, x0);
     if (kb + 1 < nkb) step(kb + 1, x1);
+    if (__builtin_amdgcn_readfirstlane(marked)) break;
+    if (bad) s_bad[group & 1] = 1;
   }
 
   // also the barrier before the buffers are reused

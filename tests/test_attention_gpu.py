@@ -258,3 +258,26 @@ def test_fp32_sizes_of_q_and_k_that_cancel(device, q_size, k_size):
     k[:, :, 9] *= 1e-3
     out = _attention_hip.attention(q.to(device), k.to(device), v.to(device), 0.125).cpu().double()
     torch.testing.assert_close(out, _f64(q, k, v, 0.125), rtol=0, atol=2.0 ** -18 * v.abs().max().item())
+
+
+@pytest.mark.parametrize('where', ['k', 'v', 'logit'])
+@pytest.mark.parametrize('at', [0, 31, 32, 63, 64, 95, 96, 128, 300, 383, 384, 415, 416])
+def test_fp32_tiles_left_at_any_key_block(device, where, at):
+    # one key that the split does not hold (or whose logits it does not), in the first blocks, at
+    # the edges of the pairs of blocks between barriers and in the last, ragged block
+    g = torch.Generator().manual_seed(at)
+    q, k, v = (torch.randn((2, 417, 64), generator=g) for _ in range(3))
+    if where == 'v':
+        v[1, at] *= 1e6
+    elif where == 'k':
+        k[1, at] *= 1e-6
+    else:
+        k[1, at] *= 40.0
+        q[1, ::50] *= 1e5
+    out = _attention_hip.attention(q.to(device), k.to(device), v.to(device), 0.125).cpu().double()
+    ref = _f64(q, k, v, 0.125)
+    if where == 'logit':     # those queries select one key; their logits' gap may be within fp32's error
+        assert torch.isfinite(out).all()
+        q, out, ref = (torch.cat([x[:, i::50] for i in range(1, 50)], 1) for x in (q, out, ref))
+    span = (q.double().norm(dim=-1).max() * k.double().norm(dim=-1).max()).item() * 0.125
+    assert ((out - ref).abs() <= 2.0 ** -20 * span * v.double().abs().amax((1, 2), keepdim=True)).all()
