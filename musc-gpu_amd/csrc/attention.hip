@@ -263,6 +263,23 @@ __device__ __forceinline__ void attend_tile_f32(float* smem, const float* __rest
   }
 }
 
+// Few keys: finding the scales and splitting cost more than the products they make cheaper.
+// us with fp32 products against the split, 16 / 64 / 512 heads: 32 keys 5.2 / 5.3 / 9.0 against
+// 6.7 / 6.9 / 13.3, 64 keys 7.8 / 8.0 / 15.0 against 7.7 / 7.9 / 15.4, 65 keys 10.4 / 10.6 / 20.6
+// against 8.9 / 9.1 / 18.2.
+constexpr int kF32Keys = 64;
+__global__ __launch_bounds__(WAVES32 * kWave, 1) void attn_fwd_short_kernel(const float* __restrict__ qg,
+                                                                            const float* __restrict__ kg,
+                                                                            const float* __restrict__ vg,
+                                                                            float* __restrict__ og, int t,
+                                                                            float scale_log2, HeadLayout in,
+                                                                            HeadLayout out, int nbh) {
+  __shared__ __attribute__((aligned(16))) float smem[kF32Smem / 4];
+  const int2 unit = fwd_unit<QW * WAVES32>(t, nbh);
+  if (unit.x < 0) return;
+  attend_tile_f32(smem, qg, kg, vg, og, t, scale_log2, in, out, unit);
+}
+
 // fp16 storage on fp16 MFMA (v_mfma_f32_32x32x16_f16): same S^T = K Q^T layout as
 // the fp32 kernel, four MFMAs per 32-key block for S (K = d = 64) and two per
 // 32-wide d tile for O^T += V^T P^T, with P rounded to fp16 (the reference feeds
@@ -1140,7 +1157,8 @@ int attention_fwd(const void* q, const void* k, const void* v, void* out, int dt
   const long long units = (long long)((t + tile - 1) / tile) * nbh;
   const dim3 grid((unsigned)align_up((size_t)units, kXcds));
   if (dtype == MUSC_DTYPE_F32)
-    hipLaunchKernelGGL(attn::attn_fwd_kernel, grid, dim3(attn::WAVES32 * kWave), 0, stream,
+    hipLaunchKernelGGL(t <= attn::kF32Keys ? attn::attn_fwd_short_kernel : attn::attn_fwd_kernel, grid,
+                       dim3(attn::WAVES32 * kWave), 0, stream,
                        static_cast<const float*>(q), static_cast<const float*>(k), static_cast<const float*>(v),
                        static_cast<float*>(out), t, scale_log2, in, ol, nbh);
   else
