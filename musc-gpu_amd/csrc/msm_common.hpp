@@ -7,6 +7,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "tile_grid.hpp"
 
 namespace musc {
 namespace msm {
@@ -57,6 +58,11 @@ __host__ __device__ inline long long band_prefix(long long s, long long T) {
 }
 
 __host__ __device__ inline long long total_tiles(long long T) { return T * (T + 1) / 2; }
+
+// This workgroup's tile number in a grid of tile_grid's.
+__device__ inline long long tile_number() {
+  return (long long)blockIdx.z * gridDim.x + xcd_logical_id(blockIdx.x, gridDim.x);
+}
 
 template <int kBand = BAND>
 __device__ inline int2 decode_tile(long long w, long long T) {

@@ -109,7 +109,7 @@ __global__ __launch_bounds__(THREADS, kSplit || kW == 1 ? 3 : 2) void msm_pair_m
   __shared__ __attribute__((aligned(16))) float s_cinv[BN];
   __shared__ int s_rimg[BM], s_cimg[BN];
 
-  const long long w = xcd_logical_id(blockIdx.x, gridDim.x);
+  const long long w = tile_number();
   if (w >= ntiles) return;
   const int2 tile = decode_tile(w, T);
   const int row0 = tile.x * BM, col0 = tile.y * BN;
@@ -540,10 +540,10 @@ int launch_pairs(const float* z, int n, int p, int c, const Workspace& w, const 
   const long long rows = (long long)n * p;
   const long long T = (rows + BM - 1) / BM;
   const long long ntiles = total_tiles(T);
-  const long long grid = (ntiles + kXcds - 1) / kXcds * kXcds;
-  if (grid > 0x7fffffffLL) return MUSC_ERR_UNSUPPORTED;
+  TileGrid grid;
+  if (!tile_grid(ntiles, THREADS, kXcds, &grid)) return MUSC_ERR_UNSUPPORTED;
 #define MUSC_PAIR_LAUNCH(V4, SPLIT)                                                                                \
-  hipLaunchKernelGGL((msm_pair_min_kernel<V4, SPLIT, kW>), dim3((unsigned)grid, pools.count), dim3(THREADS), 0, s, z, \
+  hipLaunchKernelGGL((msm_pair_min_kernel<V4, SPLIT, kW>), dim3(grid.x, pools.count, grid.z), dim3(THREADS), 0, s, z, \
                      w.norms, w.inv, w.minbits, (int)rows, n, p, c, (int)T, ntiles, pools.ws_step)
   // whole-chunk loads: c a multiple of two chunks, and a tile's panel addressable with
   // 32-bit offsets (any pool size: the buffer resources are based at each tile's panels)

@@ -223,7 +223,7 @@ __global__ __launch_bounds__(THREADS, 1) void split_pair_kernel(const _Float16* 
   __shared__ float s_cnorm[TM];
   __shared__ float s_cinv[TM];
 
-  const long long w = xcd_logical_id(blockIdx.x, gridDim.x);
+  const long long w = tile_number();
   if (w >= ntiles) return;
   const int2 tile = decode_tile<kBandSplit>(w, T);
   const int row0 = tile.x * TM, col0 = tile.y * TM;
@@ -781,10 +781,10 @@ int run_pairs(int n, int p, int c, void* ws, const Pools& pools, hipStream_t s) 
   const long long rows = (long long)n * p;
   const long long T = (rows + TM - 1) / TM;
   const long long ntiles = total_tiles(T);
-  const long long grid = (ntiles + kXcds - 1) / kXcds * kXcds;  // one workgroup per tile
-  if (grid > 0x7fffffffLL) return MUSC_ERR_UNSUPPORTED;
+  TileGrid grid;
+  if (!tile_grid(ntiles, THREADS, kXcds, &grid)) return MUSC_ERR_UNSUPPORTED;
   const Workspace w = carve(ws, n, p);
-  hipLaunchKernelGGL(split_pair_kernel, dim3((unsigned)grid, pools.count), dim3(THREADS), 0, s, split_array(ws, n, p),
+  hipLaunchKernelGGL(split_pair_kernel, dim3(grid.x, pools.count, grid.z), dim3(THREADS), 0, s, split_array(ws, n, p),
                      w.norms, w.inv, w.minbits, (int)rows, n, p, nkb_of(c), (int)T, ntiles, pools.ws_step);
   return check_launch();
 }
