@@ -18,7 +18,7 @@ namespace musc {
 namespace msm {
 
 // kW: 32 x 32 MFMA blocks per wave and dimension.  kW = 2 is the 128 x 128 tile; kW = 1 a
-// 64 x 64 tile of the same four waves, for pools whose 128-tiles leave most CUs idle.
+// 64 x 64 tile of the same four waves, for launches too small for 128-tiles (small_tile_limit).
 constexpr int tile_of(int kW) { return 64 * kW; }
 constexpr int BK = 16;           // K chunk (channels) per pipeline stage: the double-buffered
                                  // stage is 40 KB of LDS, so three workgroups share a CU
@@ -93,7 +93,7 @@ __device__ inline void store_chunk(float* __restrict__ dst, const stage4 (&reg)[
 
 // kSplit (p >= the tile): a tile's row or column range holds at most one image boundary,
 // so tiles straddling a boundary reduce in registers too, with two image segments
-// per dimension; otherwise (p < 64) they go through the LDS epilogue.
+// per dimension; otherwise they go through the LDS epilogue.
 template <int kLoad, bool kSplit, int kW>
 __global__ __launch_bounds__(THREADS, kSplit || kW == 1 ? 3 : 2) void msm_pair_min_kernel(
     const float* __restrict__ z, const float* __restrict__ norms, const float* __restrict__ inv,
@@ -550,27 +550,55 @@ int launch_pairs(const float* z, int n, int p, int c, const Workspace& w, const 
   const bool chunks = c % (2 * BK) == 0 && (unsigned long long)BM * (unsigned long long)c * 4ull < (1ull << 31);
   if (p >= BM) {
     if (chunks) MUSC_PAIR_LAUNCH(2, true); else if ((c & 3) == 0) MUSC_PAIR_LAUNCH(1, true); else MUSC_PAIR_LAUNCH(0, true);
-  } else if constexpr (kW == 1) {
+  } else {
     if (chunks) MUSC_PAIR_LAUNCH(2, false); else if ((c & 3) == 0) MUSC_PAIR_LAUNCH(1, false); else MUSC_PAIR_LAUNCH(0, false);
   }
 #undef MUSC_PAIR_LAUNCH
   return check_launch();
 }
 
-// 128-tiles need fewer operand bytes and LDS reads per MFMA, but three of them share a CU,
-// so a launch of a few thousand ends with most of its last round idle, and one below 768
-// leaves CUs empty throughout; 64-tiles are a quarter of that.  Measured by 128-tiles in the
-// launch (us, 64 against 128): 45 9.1 / 21.7, 120 21.4 / 37.8, 528 94 / 138, 820 180 / 237,
-// 1128 266 / 297, 3741 847 / 861, 5778 1277 / 1324, 7626 1751 / 1742, 8385 1404 / 1414, 11325
-// 2589 / 2545, 13861 2437 / 2363, 17020 2019 / 1971.  Patches per image below 128 always
-// take 64-tiles: a 128-tile could hold several image boundaries and reduced through LDS
-// (12403 tiles of P = 100: 2259 / 2534; P = 40, 3.96e4: 7548 / 8060).  Both tiles add a
-// dot product's terms in the same order: the same bits.
-constexpr long long kSmallTiles = 6000;
+// Number of 128-tiles of a launch (over all its pools) below which it takes 64-tiles.
+// 128-tiles need fewer operand bytes and LDS reads per MFMA, but three of them share a CU, so
+// a launch of a few hundred leaves CUs empty and one of a thousand ends with most of its last
+// round idle; 64-tiles are a quarter of that.  Both tiles add a dot product's terms in the same
+// order: the same bits.  Measured (us, 64 against 128, by number of 128-tiles):
+//   P >= 128, whole chunks, C = 1024: 253 70 / 74, 561 128 / 184, 1176 282 / 300, 2145 487 / 525,
+//     2628 654 / 638, 3240 799 / 762, 5886 1430 / 1337; C = 384: 1176 113 / 120, 2080 197 / 208,
+//     3240 305 / 300, 5886 577 / 526.  P = 1369, C = 1024: 2850 659 / 688, 4753 1068 / 1082, 5778
+//     1347 / 1328; 3741 863 / 860 launched over and over, in a division of 8 images as a whole
+//     916 / 932.
+//   Few channels (the epilogue is most of a tile): C = 64 820 25.0 / 26.8, 1176 34.6 / 32.1;
+//     C = 32 136 5.8 / 6.7, 406 11.9 / 10.7, 1176 29.6 / 22.6.
+//   C % 4 = 0 (masked loads): C = 1020 946 260 / 278, 1485 399 / 385, 2080 599 / 574; C = 388 1176
+//     137 / 143, 2628 310 / 291.
+//   Other C (scalar loads, which a 64-tile issues twice as often per product): C = 1021 136 126 /
+//     129, 253 163 / 129, 1176 702 / 552; C = 201 253 34 / 30, 1176 129 / 112; C = 101 528 38 / 41,
+//     1176 72 / 66.
+//   P < 128, where a 128-tile may hold several image boundaries and reduces through LDS, a
+//     64-tile from P = 64 on in registers: C = 1024 P = 100 2145 558 / 603, 19306 4885 / 5047; P =
+//     49 11935 3108 / 3133; C = 64 P = 100 27730 1062 / 1192, P = 49 1081 70 / 76, 1953 115 / 110;
+//     C = 1020 P = 100 3160 924 / 993, 4465 1328 / 1288, P = 49 1953 581 / 588, 3003 912 / 879;
+//     C = 700 P = 100 7875 1621 / 1642; C = 1021 P = 100 300 209 / 243, 1128 706 / 582; C = 301 528
+//     90 / 118, 1128 190 / 187, 2145 353 / 321; C = 101 7875 484 / 586; P = 9 C = 384 946 220 / 213.
+constexpr long long kAllSmall = 1LL << 60;
+inline long long small_tile_limit(int p, int c) {
+  const bool whole = c % (2 * BK) == 0, vec = c % 4 == 0;
+  if (p >= tile_of(2)) {
+    if (c <= 64) return c <= 32 ? 300 : 1000;
+    if (whole) return p < 1024 ? 2400 : 5000;
+    if (vec) return 1400;
+    return c < 128 ? 700 : 192;
+  }
+  if (!vec) return c < 128 ? kAllSmall : 300000 / c;
+  if (p < 32 || (p < tile_of(1) && c <= 64)) return 1500;
+  if (whole || c <= 768) return kAllSmall;
+  return p < tile_of(1) ? 2000 : 3500;
+}
+
 int run_pairs(const float* z, int n, int p, int c, const Workspace& w, const Pools& pools, hipStream_t s) {
   const long long T = ((long long)n * p + tile_of(2) - 1) / tile_of(2);
-  return p < tile_of(2) || total_tiles(T) * pools.count < kSmallTiles ? launch_pairs<1>(z, n, p, c, w, pools, s)
-                                                                      : launch_pairs<2>(z, n, p, c, w, pools, s);
+  return total_tiles(T) * pools.count < small_tile_limit(p, c) ? launch_pairs<1>(z, n, p, c, w, pools, s)
+                                                               : launch_pairs<2>(z, n, p, c, w, pools, s);
 }
 
 }  // namespace msm

@@ -217,3 +217,27 @@ def test_both_tiles_of_the_pair_kernel_agree(device, n, p, c):
                 assert torch.equal(many[0, k].view(torch.int64), one[0, 0].view(torch.int64)), k
     finally:
         pipeline.POOLS_WORKSPACE = before
+
+
+@pytest.mark.parametrize('n,p,c,pools', [(5, 100, 1021, 60), (9, 100, 301, 60), (7, 127, 201, 80), (9, 64, 1023, 60),
+                                         (9, 49, 64, 200), (9, 63, 32, 200), (60, 7, 384, 180), (40, 1, 1020, 1600),
+                                         (10, 49, 1020, 200), (8, 100, 1020, 130), (12, 31, 33, 700)])
+def test_both_tiles_agree_with_few_patches_per_image(device, n, p, c, pools):
+    # P < 128: the 128-tile holds several image boundaries per dimension and reduces through LDS,
+    # the 64-tile of a single pool does so below P = 64; enough pools in a launch to take 128-tiles
+    # (the last shape stays with 64-tiles).  The same bits, and one pool against the oracle
+    g = torch.Generator(device='cuda').manual_seed(n * p + c)
+    z = torch.randn((1, pools, n, p, c), generator=g, device=device)
+    z[0, 1, 1, 0] = z[0, 1, 0, p - 1]
+    z[0, 2, 0, 0, 0] = float('nan')
+    before, pipeline.POOLS_WORKSPACE = pipeline.POOLS_WORKSPACE, 8 << 30
+    try:
+        many = pipeline.msm_all(z, topmin_max=1)
+        for k in [1, 2] + list(range(0, pools, max(1, pools // 6))):
+            one = pipeline.msm_all(z[:, k:k + 1], topmin_max=1)
+            assert torch.equal(many[0, k].view(torch.int64), one[0, 0].view(torch.int64)), k
+    finally:
+        pipeline.POOLS_WORKSPACE = before
+    last = z[0, pools - 1].cpu()
+    ref = om.MSM(last / last.norm(dim=-1, keepdim=True), 0, 1).numpy()   # msm_all normalises the rows
+    assert np.abs(many[0, pools - 1].cpu().numpy() - ref).max() <= ATOL
