@@ -34,6 +34,7 @@ from . import _runtime as rt
 # Workspace of one launch over several pools: the reference's own scratch cap
 # (models/modules/_MSM_gpu.py:11).  Larger pools are scored one at a time.
 POOLS_WORKSPACE = 256 << 20
+POOLS_PER_LAUNCH = 65535      # pools are a grid dimension
 
 
 def lnamd_pools(tokens: list[torch.Tensor], r_list: list[int], pool_grid: int | None = None) -> torch.Tensor:
@@ -77,7 +78,7 @@ def msm_all(pools: torch.Tensor, topmin_min: float = 0, topmin_max: float = 0.3,
         per_pool = _MSM_hip.workspace_bytes(n, p, c, engine)
         s = rt.stream(pools.device)
         if pair_events is None and rank_events is None and refine_events is None:
-            group = min(r * l, max(1, POOLS_WORKSPACE // per_pool))
+            group = max(1, min(r * l, POOLS_WORKSPACE // per_pool, POOLS_PER_LAUNCH))
             ws = rt.workspace(group * per_pool, pools.device)
             z_step, s_step = n * p * c * 4, n * p * 8
             for k in range(0, r * l, group):

@@ -92,3 +92,19 @@ def test_pools_in_one_launch_match_pool_by_pool(device, monkeypatch, engine, r, 
         got = pipeline.msm_all(z, normalize_rows=normalize, engine=engine, **window)
         ref = pipeline.msm_all(z, normalize_rows=normalize, engine=engine, pair_events=[], **window)
         assert torch.equal(got.view(torch.int64), ref.view(torch.int64))
+
+
+@pytest.mark.parametrize('engine,p', [('fp32', 9), ('split16', 256)])
+@pytest.mark.parametrize('r,l', [(0, 2), (2, 0), (0, 0)])
+def test_no_pools_give_no_scores(device, engine, p, r, l):
+    got = pipeline.msm_all(torch.empty((r, l, 5, p, 8), device=device), engine=engine)
+    assert got.shape == (r, l, 5, p) and got.dtype == torch.float64 and got.device.type == 'cuda'
+
+
+def test_more_pools_than_a_grid_dimension_holds(device):
+    g = torch.Generator().manual_seed(2)
+    z = torch.randn((70, 1000, 2, 1, 4), generator=g)
+    got = pipeline.msm_all(z.to(device), topmin_max=1.0)
+    u = z.double() / z.double().norm(dim=-1, keepdim=True)
+    ref = (u[:, :, 0] - u[:, :, 1]).norm(dim=-1)[:, :, None].expand(-1, -1, 2, -1)
+    assert (got.cpu() - ref).abs().max() <= ATOL
