@@ -19,7 +19,7 @@
 // non-negative number as unsigned integers, so the atomic keeps them too.
 //
 // Bound by the float64 map writes: N = 83, 3 x 4 maps, 37 -> 518 (178 MB written, 11 MB
-// read) in 36.6 us = 5.2 TB/s, the rate of a large copy; 62.5 us when every pixel formed
+// read) in 37.8 us = 5.0 TB/s, the rate of a large copy; 62.5 us when every pixel formed
 // its own coordinates and both horizontal interpolants in 8-row bands.
 #include "common.hpp"
 
@@ -34,6 +34,9 @@ constexpr int kFillBlocks = 256;   // workgroups wanted before bands grow (one p
 
 __device__ inline double nmax(double a, double b) { return __builtin_elementwise_maximum(a, b); }
 
+// kGroups > 1 (rows narrower than a workgroup): that many groups of blockDim.x / kGroups
+// threads, each with a column per thread, walk equal runs of the band's rows.
+template <int kGroups>
 __global__ __launch_bounds__(kMaxThreads) void maps_kernel(const double* __restrict__ scores, int n_radii,
                                                            int n_layers, int n, int side, int out_size, int rows,
                                                            double* __restrict__ maps,
@@ -72,22 +75,26 @@ __global__ __launch_bounds__(kMaxThreads) void maps_kernel(const double* __restr
   }
   __syncthreads();
 
+  constexpr int kCols = 4 * kWave / kGroups;  // columns of a group
+  const int per = (y1 - y0 + kGroups - 1) / kGroups;
+  const int yb = kGroups > 1 ? (int)threadIdx.x / kCols * per : 0, ye = kGroups > 1 ? min(yb + per, y1 - y0) : y1 - y0;
+  const int first = kGroups > 1 ? (yb < ye ? (int)threadIdx.x % kCols : out_size) : (int)threadIdx.x;
   double vmax = 0.0;
-  for (int x = threadIdx.x; x < out_size; x += blockDim.x) {
+  for (int x = first; x < out_size; x += blockDim.x) {
     const double sx = scale * x;
     const int w0 = (int)sx;
     const int w1 = w0 < side - 1 ? w0 + 1 : w0;
     const double lw1 = sx - w0, lw0 = 1.0 - lw1;
     auto across = [&](int g) { return lw0 * avg[g - g0][w0] + lw1 * avg[g - g0][w1]; };
     double* dst = maps ? maps + ((long long)img * out_size + y0) * out_size + x : nullptr;
-    int h = s_h0[0];                      // grid row of `top`; the same in every thread
+    int h = s_h0[yb];                     // grid row of `top`; the same in every thread of a group
     double top = across(h), bottom = across(min(h + 1, side - 1));
     int next_h0 = h;                      // the next output row's table entries, read one row ahead
-    double next_lh1 = s_lh1[0];
-    for (int y = 0; y < y1 - y0; ++y) {
+    double next_lh1 = s_lh1[yb];
+    for (int y = yb; y < ye; ++y) {
       const int h0 = next_h0;
       const double lh1 = next_lh1, lh0 = 1.0 - lh1;
-      const int yn = min(y + 1, y1 - y0 - 1);
+      const int yn = min(y + 1, ye - 1);
       next_h0 = s_h0[yn];
       next_lh1 = s_lh1[yn];
       if (h0 != h) {
@@ -135,15 +142,23 @@ extern "C" int musc_maps_f64(const double* scores, int n_radii, int n_layers, in
   // neighbours; 16-row bands only where 32 would leave CUs idle (3 x 4 maps, 37 -> 518, by
   // N, 16 against 32 rows: N = 8 12.0 / 12.8 us, 16 15.9 / 15.7, 83 42.5 / 37.8)
   if (rows > 16 && (long long)n * ((out_size + rows - 1) / rows) < epi::kFillBlocks) rows = 16;
-  // a handful of small maps: the walk down a band is all the time there is
+  // a handful of small maps: the walk down a band is all the time there is (one image, 3 x 4 maps,
+  // 37 -> 518, 8 against 16 rows: 7.4 / 8.1 us; 8 images 64 -> 64 5.8 / 6.3; 14 -> 100 5.9 / 5.7)
   if (rows > 8 && (long long)n * ((out_size + rows - 1) / rows) < epi::kFillBlocks / 4) rows = 8;
   const int bands = (out_size + rows - 1) / rows;
-  // a column per thread; at least four waves for the averaging
+  // a column per thread; at least four waves, for the averaging and, on rows of up to 128 columns,
+  // in groups that share the band's rows (one map, 83 images 64 -> 64: 8.4 us with three of four
+  // waves idle, 7.1 so; 16 -> 128: 9.9 / 8.2; 500 of 8 -> 16: 7.0 / 5.4).  A last turn of few
+  // columns past 1024 stays: equal turns, with fewer waves, take 188 us for 1030 where it takes 166
   const int threads = min(max((out_size + kWave - 1) / kWave * kWave, 4 * kWave), epi::kMaxThreads);
   if ((long long)n * bands > 0x7fffffffLL) return MUSC_ERR_UNSUPPORTED;
   unsigned long long* bits = reinterpret_cast<unsigned long long*>(image_scores);
   if (bits) launch_fill_u32(reinterpret_cast<uint32_t*>(bits), (size_t)n * 2, 0u, stream);
-  hipLaunchKernelGGL(epi::maps_kernel, dim3((unsigned)(n * bands)), dim3(threads), 0, stream, scores, n_radii,
-                     n_layers, n, side, out_size, rows, maps, bits);
+  auto kernel = epi::maps_kernel<1>;
+  if (out_size <= kWave / 2) kernel = epi::maps_kernel<8>;
+  else if (out_size <= kWave) kernel = epi::maps_kernel<4>;
+  else if (out_size <= 2 * kWave) kernel = epi::maps_kernel<2>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(n * bands)), dim3(threads), 0, stream, scores, n_radii, n_layers, n, side,
+                     out_size, rows, maps, bits);
   return check_launch();
 }

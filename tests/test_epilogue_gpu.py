@@ -56,3 +56,16 @@ def test_band_heights_and_wide_rows(device, n, side, size):
     ref_maps, ref_img = oe.maps_and_scores([[torch.from_numpy(raw[0, l]) for l in range(2)]], size)
     np.testing.assert_allclose(maps.cpu().numpy(), ref_maps.numpy(), rtol=0, atol=1e-12)
     np.testing.assert_allclose(img.cpu().numpy(), ref_img.numpy(), rtol=0, atol=1e-12)
+
+
+@pytest.mark.parametrize('n', [1, 8, 83])
+@pytest.mark.parametrize('side,size', [(3, 1), (4, 2), (5, 7), (12, 31), (12, 32), (6, 33), (14, 63), (14, 64), (9, 65),
+                                       (20, 100), (37, 127), (16, 128), (16, 129), (100, 33), (128, 9)])
+def test_narrow_maps(device, n, side, size):
+    # rows of up to 32, 64 and 128 columns, whose bands are shared by groups of threads
+    rng = np.random.default_rng(n * 1000 + size)
+    raw = rng.random((2, 1, n, side * side))
+    maps, img = _epilogue_hip.maps_and_scores(torch.from_numpy(raw).to(device), size)
+    ref_maps, ref_img = oe.maps_and_scores([[torch.from_numpy(raw[r, 0])] for r in range(2)], size)
+    np.testing.assert_allclose(maps.cpu().numpy(), ref_maps.numpy(), rtol=0, atol=1e-12)
+    np.testing.assert_allclose(img.cpu().numpy(), ref_img.numpy(), rtol=0, atol=1e-12)
