@@ -418,7 +418,7 @@ struct Plan {
   AxisGeom gh, gv;
   bool need_h, need_v;
   TilePlan tile;             // fused kernel, when tile.band > 0
-  bool words;                // images must be 4-byte aligned, and no uint8 intermediate is reserved
+  bool words;                // the interface asks for 4-byte aligned images and reserves no uint8 intermediate
   int width;                 // coefficient row width (both axes): a bucket >= the taps of either axis
   int taps;                  // the larger of the two axes' tap counts
   int row0, rows;            // source rows the vertical pass reads (horizontal pass extent)
@@ -437,7 +437,8 @@ inline Plan plan(int batch, int in_h, int in_w, int out_h, int out_w) {
   p.width = table_width(p.taps);
   const bool both = p.need_h && p.need_v;
   p.tile = both ? tile_plan(batch, in_h, in_w, out_h, out_w, p.gh, p.gv, p.taps) : TilePlan{0, 0, 0, 0, 0};
-  // what the interface states; the fused kernel itself takes other widths and alignments too
+  // the terms of the interface, which callers size and align their buffers by; the fused kernel
+  // itself takes other widths, alignments and tap counts too and then leaves the room unused
   p.words = both && in_w % 4 == 0 && out_w <= 768 && p.taps <= 15;
   if (p.need_h && p.need_v) {
     const int2 first = window(p.gv, in_h, 0, nullptr);
@@ -458,7 +459,8 @@ inline Plan plan(int batch, int in_h, int in_w, int out_h, int out_w) {
   p.off_kv = off;
   off = align_up(off + (size_t)out_h * p.width * sizeof(int), 256);
   p.off_tmp = off;
-  if (p.need_h && !p.words) off = align_up(off + (size_t)batch * p.rows * out_w * 3, 256);
+  // the two passes write an intermediate: whoever takes them has room for it
+  if (p.need_h && (!p.words || p.tile.band == 0)) off = align_up(off + (size_t)batch * p.rows * out_w * 3, 256);
   p.total = off;
   return p;
 }

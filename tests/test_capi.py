@@ -4,7 +4,9 @@ Only argument-validation paths are called here: each returns its error code
 before any HIP call, so no GPU is touched.
 """
 import ctypes
+import math
 import os
+import random
 import re
 
 import pytest
@@ -201,3 +203,30 @@ def test_msm_pools_argument_errors(lib):
     assert call(pools=70000) == 1003 and call(engine=1, p=100) == 1003 and call(n=5000, p=1) == 1003
     assert lib.musc_msm_workspace_bytes(8, 300, 16, ctypes.byref(one)) == 0
     assert call(size=ctypes.c_size_t(2 * one.value - 1)) == 1002
+
+
+def test_preprocess_without_an_intermediate_always_fuses(lib):
+    # sizes whose workspace holds the two tables only (both axes resampled, in_w % 4 == 0, out_w <=
+    # 768, at most 15 taps) must take the fused kernel: the two passes write an intermediate, which
+    # the size would then include
+    align = lambda x: (x + 255) // 256 * 256  # noqa: E731
+    taps = lambda a, b: 2 * math.ceil(2.0 * max(a / b, 1.0)) + 1  # noqa: E731
+    rng = random.Random(0)
+    sizes = [(1, 1, 4, 1, 1), (1, 1, 4, 65535, 1), (1, 65535, 4, 20000, 768), (65535, 9, 2628, 3, 768), (1, 9, 2684, 9, 767),
+             (1, 2690, 2688, 768, 768), (3, 8, 8, 65535, 768), (1, 60000, 4, 65535, 5)]
+    for _ in range(3000):
+        out_h, out_w = int(2 ** rng.uniform(0, 12)), int(2 ** rng.uniform(0, 9.58))
+        in_h = max(1, int(out_h * 2 ** rng.uniform(-6, 1.8)))
+        in_w = max(1, int(out_w * 2 ** rng.uniform(-6, 1.8)) // 4) * 4
+        sizes.append((rng.choice([1, 3, 64]), in_h, in_w, out_h, out_w))
+    out, seen = ctypes.c_size_t(), 0
+    for b, in_h, in_w, out_h, out_w in sizes:
+        t = max(taps(in_h, out_h), taps(in_w, out_w))
+        if in_h == out_h or in_w == out_w or t > 15:
+            continue
+        width = next(w for w in (4, 8, 12, 16) if t <= w)
+        assert lib.musc_preprocess_workspace_bytes(b, in_h, in_w, out_h, out_w, ctypes.byref(out)) == 0
+        tables = sum(align(n * 8) + align(n * width * 4) for n in (out_w, out_h))
+        assert out.value == tables, (b, in_h, in_w, out_h, out_w)
+        seen += 1
+    assert seen > 2000
