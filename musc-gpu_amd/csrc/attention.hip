@@ -320,8 +320,11 @@ constexpr int VR16 = D + 8;        // V block pitch (halves), row-major: 144 B r
 // first and the last runs alone.  Waves 0-7 stage: one float4 of K and one of V per
 // thread and 32-key block, loaded two blocks before they are split into LDS, which
 // happens while the logits' MFMAs run; a barrier every kGroup blocks.
-//   Bound by MFMA issue: B = 4, H = 16, T = 1370 (24 MFMAs, about 112 VALU instructions
-// per wave and block) 97 us = 317 TFLOP/s in fp32 terms; the fp32 MFMA tiles took 266 us
+//   Bound by MFMAs and VALU work that take turns: B = 4, H = 16, T = 1370 (per wave and
+// block 24 MFMAs and, staging included, 158 other VALU instructions) 94-98 us = 314-327 TFLOP/s
+// in fp32 terms, the MFMA pipe busy for 43 % of the cycles and the VALU for 46 %; the three
+// waves of a SIMD, in step at the barriers, overlap the two little (34 % of wave cycles wait
+// for an issue slot, 37 % for LDS, memory or the barrier).  The fp32 MFMA tiles took 266 us
 // (116 TFLOP/s, 74 % of the fp32 peak).  Timing-only copies: 4 of the 24 MFMAs less
 // -12 %, no staging -8 %, no exponentials -6 %, no split of P -5 %, no maximum -1 %.
 // Measured and not kept: one block per barrier 102 us, four 97 us; the next block's

@@ -19,10 +19,11 @@
 //                          column in a register ring, puts the nested vertical sums
 //                          of each output row in LDS (double-buffered, one barrier
 //                          per row) and adds its horizontal neighbours'.  Every
-//                          token is read once, every output written once.  Where the
-//                          columns alone do not fill the chip (a few images), they are
-//                          split into bands of rows: a whole column is 37 dependent
-//                          rows long whatever the batch.
+//                          output is written once, every token read once, except
+//                          where the columns alone do not fill the chip (a few
+//                          images): they are split into bands of rows there (a whole
+//                          column is 37 dependent rows long whatever the batch), which
+//                          read the 2*hmax rows around them as well.
 //   lnamd_pool_kernel      L2-normalising path.  One workgroup per (image, layer, output row); each
 //                          thread owns 4 channels.  It sweeps the row's columns,
 //                          reading the 2*hmax+1 input rows once per column, keeps
@@ -72,8 +73,8 @@ __device__ inline float4 load4(const void* base, long long idx4) {
   }
 }
 
-// Same as load4 with the nontemporal hint, for tokens a kernel reads exactly once
-// (statistics pass, streaming pass): +20 % on the statistics pass, measured.
+// Same as load4 with the nontemporal hint, for the passes that read the tokens once or, with
+// bands of rows, little more (statistics, streaming): +20 % on the statistics pass, measured.
 typedef float nt_load_f4 __attribute__((ext_vector_type(4)));
 typedef unsigned int nt_load_u2 __attribute__((ext_vector_type(2)));
 template <int kDtype>

@@ -23,7 +23,7 @@
 // layers and radii go through one launch per stage, because a few small images leave most
 // of the chip idle in each launch (45 workgroups of the pair kernel for one pool of eight
 // 12 x 12 images): tokens to maps of eight such images, two layers and two radii, 168.6 us
-// pool by pool (29 launches), 65.3 us together (10).
+// pool by pool (29 launches), 64.2 us together (10).
 #include <mutex>
 
 #include "msm_common.hpp"

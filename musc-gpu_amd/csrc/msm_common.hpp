@@ -188,8 +188,9 @@ inline size_t workspace_bytes(long long n, long long p) {
   return 3 * align_up((size_t)rows * 4, 256) + align_up((size_t)rows * n * 4, 256) + align_up((size_t)n * 4, 256);
 }
 
-// A launch over several pools of one shape: gridDim.y pools, pool k's features z + k * z_step
-// and workspace `ws_step` bytes after pool k - 1's (both 0 for one pool).
+// A launch over several pools of one shape, gridDim.y of them: pool k's features begin at
+// z + k * rows * c (the pools are contiguous), its workspace `ws_step` bytes after pool
+// k - 1's (0 for one pool).
 struct Pools {
   int count;
   size_t ws_step;

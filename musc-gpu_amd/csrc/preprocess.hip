@@ -204,7 +204,8 @@ __global__ __launch_bounds__(kThreads) void vpass_kernel(const uint8_t* __restri
 // and the uint8 intermediate never reaches HBM.  Any in_w and image alignment: a row's
 // words start at its address rounded down to 4, the remainder joins the window's offset.
 // Bound by instruction issue (a byte extraction and a 24-bit multiply-add per tap and
-// channel) and, up to four images, by the host and the launches.  Whole call, 1024 x 1024 ->
+// channel: the VALU is busy for 96 % of the cycles) and, up to four images, by the host and the
+// launches.  Whole call, 1024 x 1024 ->
 // 518: one image 48.9 -> 18.2 us, 4 51.9 -> 18.6, 16 97.1 -> 42.9 against a band of 8 whole rows per
 // workgroup, its source rows staged one at a time with a barrier each; 4 of 1023 x 1023, whose
 // width took two passes through HBM, 56.9 -> 18.6.  With a test of every word
