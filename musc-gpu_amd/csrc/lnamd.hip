@@ -354,8 +354,10 @@ __global__ __launch_bounds__(kMaxThreads) void lnamd_pool_kernel(TokenPtrs token
 // sums accumulate in two register slots (a source row lies in at most two output
 // windows when pool <= side); an output row is written when its last source row
 // is done.  raw = 0 divides by r^2 and the window count, raw = 1 writes the plain
-// sums.
-template <int kDtype, int kHalo, int kNR, bool kPool>
+// sums.  kBands: the columns are split into bands of `band` rows; without, the loop starts at
+// row 0 for the compiler too, which peels the rows before the first output (83 images, r = 9,
+// 316 us as one kernel with the bands, 309 so).
+template <int kDtype, int kHalo, int kNR, bool kPool, bool kBands>
 __global__ __launch_bounds__(1024) void lnamd_stream_kernel(TokenPtrs tokens, int n_layers, int batch,
                                                             int tokens_per_image, int c, int has_cls, int side,
                                                             int cg, int slices, Radii radii, Radii slot, int raw,
@@ -365,11 +367,13 @@ __global__ __launch_bounds__(1024) void lnamd_stream_kernel(TokenPtrs tokens, in
   extern __shared__ float4 vsum[];  // [2][kNR][side * cg], then (kPool) hsum [kNR][side * cg]
   // XCD-grouped order: the slices of one (image, layer) run on one XCD (-3 % time
   // at config 2, measured).  The grid is padded to a multiple of kXcds.
-  const long long wid = xcd_logical_id(blockIdx.x, gridDim.x);
-  const int bands = (side + band - 1) / band;
-  if (wid >= (long long)batch * n_layers * slices * bands) return;
-  const int slice = (int)(wid % slices), unit = (int)(wid / slices / bands);
-  const int h0 = (int)(wid / slices % bands) * band, h1 = min(h0 + band, side);  // this workgroup's output rows
+  // (32 bits: the host keeps the grid in an int)
+  const unsigned wid = (unsigned)xcd_logical_id(blockIdx.x, gridDim.x);
+  const unsigned bands = kBands ? (unsigned)(side + band - 1) / band : 1u, column = wid / slices;
+  if (wid >= (unsigned)batch * n_layers * slices * bands) return;
+  const int slice = (int)(wid % slices), unit = (int)(column / bands);
+  // this workgroup's output rows
+  const int h0 = kBands ? (int)(column % bands) * band : 0, h1 = kBands ? min(h0 + band, side) : side;
   const int b = unit / n_layers, l = unit % n_layers;
   const int w = threadIdx.x / cg, gl = threadIdx.x % cg;
   const int groups = c / 4;
@@ -393,7 +397,7 @@ __global__ __launch_bounds__(1024) void lnamd_stream_kernel(TokenPtrs tokens, in
   float4 ring[2 * kHalo + 1];
 #pragma unroll
   for (int i = 0; i < 2 * kHalo + 1; ++i) ring[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-  const int first = max(h0 - kHalo, 0), end = min(h1 + kHalo, side);  // source rows
+  const int first = kBands ? max(h0 - kHalo, 0) : 0, end = kBands ? min(h1 + kHalo, side) : side;  // source rows
   float4 next = load4_once<kDtype>(base, col_base4 + (long long)first * row_step4);
 
   for (int hi = first; hi < h1 + kHalo; ++hi) {
@@ -504,13 +508,13 @@ __global__ __launch_bounds__(1024) void lnamd_stream_kernel(TokenPtrs tokens, in
   }
 }
 
-template <int kDtype, int kHalo, bool kPool>
+template <int kDtype, int kHalo, bool kPool, bool kBands>
 int dispatch_stream_nr(int nr, dim3 grid, dim3 block, size_t smem, hipStream_t s, const TokenPtrs& tp, int n_layers,
                        int batch, int tpi, int c, int has_cls, int side, int cg, int slices, const Radii& radii,
                        const Radii& slot, int raw, int layout, int pool, int band, const double* stats, float* out) {
 #define MUSC_STREAM_CASE(NR)                                                                                      \
   case NR:                                                                                                        \
-    hipLaunchKernelGGL((lnamd_stream_kernel<kDtype, kHalo, NR, kPool>), grid, block, smem, s, tp, n_layers, batch, \
+    hipLaunchKernelGGL((lnamd_stream_kernel<kDtype, kHalo, NR, kPool, kBands>), grid, block, smem, s, tp, n_layers, batch, \
                        tpi, c, has_cls, side, cg, slices, radii, slot, raw, layout, pool, band, stats, out);      \
     break;
   switch (nr) {
@@ -531,8 +535,13 @@ int dispatch_stream(int halo, int nr, dim3 grid, dim3 block, size_t smem, hipStr
                     float* out) {
 #define MUSC_STREAM_HALO(H)                                                                                      \
   case H:                                                                                                        \
-    return dispatch_stream_nr<kDtype, H, kPool>(nr, grid, block, smem, s, tp, n_layers, batch, tpi, c, has_cls,   \
-                                                side, cg, slices, radii, slot, raw, layout, pool, band, stats, out);
+    return band < side && !kPool                                                                                  \
+               ? dispatch_stream_nr<kDtype, H, false, true>(nr, grid, block, smem, s, tp, n_layers, batch, tpi, c,  \
+                                                            has_cls, side, cg, slices, radii, slot, raw, layout,    \
+                                                            pool, band, stats, out)                                \
+               : dispatch_stream_nr<kDtype, H, kPool, false>(nr, grid, block, smem, s, tp, n_layers, batch, tpi, c, \
+                                                             has_cls, side, cg, slices, radii, slot, raw, layout,   \
+                                                             pool, band, stats, out);
   switch (halo) {
     MUSC_STREAM_HALO(0)
     MUSC_STREAM_HALO(1)
@@ -727,15 +736,21 @@ int lnamd_run(const void* const* tokens, int n_layers, int in_dtype, int batch, 
     // Rows per workgroup: the whole column where the grid fills the chip; a few images are
     // split into bands, which read their 2 * halo neighbouring rows again (from L2) but
     // sweep fewer rows one after the other.  Pooling sums across rows and is not split.
-    // Whole call with and without bands (37 x 37 x 1024 fp32): 3 images, r = 1, 24.6 against
-    // 72.8 us; 8 images 36.2 / 81.0; 8 images, r = 1, 3, 5, 58.9 / 112.5; 16 images 94.0 /
-    // 133.7 (the statistics pass' share included).
+    // Stopped before the bands take a second turn on the chip: that costs more than the shorter
+    // sweep gives.  Whole calls with and without bands (37 x 37 x 1024, 16 columns' workgroups per
+    // image, three on a CU): 8 images, r = 1, 3, 5, 57 against 84 us; 16 images (512
+    // workgroups split) 92 / 106, r = 7, 9 88 / 115; 20 (640) 132 / 131, fp16 120 / 132; 24 (768) 147 /
+    // 145, fp16 131 / 143; 26 (832) 178 / 154, r = 7, 9 180 / 149; 31 (992) 192 / 173, 192 / 153.
     int band = side;
     const int least = halo < 1 ? 4 : 4 * halo;
-    if (!pooled)
-      while (band > least && (long long)units * slices * ((side + band - 1) / band) < kStreamGrid)
-        band = band / 2 > least ? (band + 1) / 2 : least;
-    const long long work = (long long)units * slices * ((side + band - 1) / band);
+    auto work_of = [&](int rows) { return (long long)units * slices * ((side + rows - 1) / rows); };
+    const long long resident = 256 * (32 / ((threads + kWave - 1) / kWave));  // workgroups the chip holds by waves
+    while (!pooled && band > least && work_of(band) < kStreamGrid) {
+      const int less = band / 2 > least ? (band + 1) / 2 : least;
+      if (work_of(less) > resident) break;
+      band = less;
+    }
+    const long long work = work_of(band);
     const dim3 grid((unsigned)((work + kXcds - 1) / kXcds * kXcds));
     const int pool = pooled ? pool_side : side;
     if (in_dtype == MUSC_DTYPE_F32)
