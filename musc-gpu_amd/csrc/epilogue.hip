@@ -67,7 +67,7 @@ __global__ __launch_bounds__(kMaxThreads) void maps_kernel(const double* __restr
     }
     avg[t / side][gc] = rsum / (double)n_radii;
   }
-  if (threadIdx.x < y1 - y0) {
+  if (kGroups == 1 && threadIdx.x < y1 - y0) {
     const double sy = scale * (y0 + (int)threadIdx.x);
     const int h0 = (int)sy;
     s_h0[threadIdx.x] = h0;
@@ -87,16 +87,24 @@ __global__ __launch_bounds__(kMaxThreads) void maps_kernel(const double* __restr
     const double lw1 = sx - w0, lw0 = 1.0 - lw1;
     auto across = [&](int g) { return lw0 * avg[g - g0][w0] + lw1 * avg[g - g0][w1]; };
     double* dst = maps ? maps + ((long long)img * out_size + y0) * out_size + x : nullptr;
-    int h = s_h0[yb];                     // grid row of `top`; the same in every thread of a group
+    // a group's few rows form their coordinates themselves, a whole band reads the table
+    int h = kGroups > 1 ? (int)(scale * (y0 + yb)) : s_h0[0];  // grid row of `top`; the same throughout a group
     double top = across(h), bottom = across(min(h + 1, side - 1));
     int next_h0 = h;                      // the next output row's table entries, read one row ahead
-    double next_lh1 = s_lh1[yb];
+    double next_lh1 = kGroups > 1 ? 0.0 : s_lh1[0];
     for (int y = yb; y < ye; ++y) {
-      const int h0 = next_h0;
-      const double lh1 = next_lh1, lh0 = 1.0 - lh1;
-      const int yn = min(y + 1, ye - 1);
-      next_h0 = s_h0[yn];
-      next_lh1 = s_lh1[yn];
+      int h0 = next_h0;
+      double lh1 = next_lh1;
+      if constexpr (kGroups > 1) {
+        const double sy = scale * (y0 + y);
+        h0 = (int)sy;
+        lh1 = sy - h0;
+      } else {
+        const int yn = min(y + 1, ye - 1);
+        next_h0 = s_h0[yn];
+        next_lh1 = s_lh1[yn];
+      }
+      const double lh0 = 1.0 - lh1;
       if (h0 != h) {
         top = h0 == h + 1 ? bottom : across(h0);
         bottom = across(min(h0 + 1, side - 1));
@@ -116,7 +124,7 @@ __global__ __launch_bounds__(kMaxThreads) void maps_kernel(const double* __restr
     __syncthreads();
     if (threadIdx.x == 0) {
       double m = wmax[0];
-      for (int w = 1; w < (int)(blockDim.x / kWave); ++w) m = nmax(m, wmax[w]);
+      for (int w = 1; w < (kGroups > 1 ? 4 : (int)(blockDim.x / kWave)); ++w) m = nmax(m, wmax[w]);
       atomicMax(image_bits + img, (unsigned long long)__double_as_longlong(m));
     }
   }
@@ -141,10 +149,14 @@ extern "C" int musc_maps_f64(const double* scores, int n_radii, int n_layers, in
   // 32-row bands repeat less of the averaging of the grid rows shared with their
   // neighbours; 16-row bands only where 32 would leave CUs idle (3 x 4 maps, 37 -> 518, by
   // N, 16 against 32 rows: N = 8 12.0 / 12.8 us, 16 15.9 / 15.7, 83 42.5 / 37.8)
-  if (rows > 16 && (long long)n * ((out_size + rows - 1) / rows) < epi::kFillBlocks) rows = 16;
+  // (upsampling less than four times, where the averaging is most of the work, four times the
+  // workgroups before 32 rows, eight before 16: 25 maps 125 -> 140 10.9 us without, 9.5 so)
+  const bool wide = scale < 0.25;
+  auto blocks = [&](int r) { return (long long)n * ((out_size + r - 1) / r); };
+  if (rows > 16 && blocks(rows) < (wide ? 1 : 4) * epi::kFillBlocks) rows = 16;
   // a handful of small maps: the walk down a band is all the time there is (one image, 3 x 4 maps,
   // 37 -> 518, 8 against 16 rows: 7.4 / 8.1 us; 8 images 64 -> 64 5.8 / 6.3; 14 -> 100 5.9 / 5.7)
-  if (rows > 8 && (long long)n * ((out_size + rows - 1) / rows) < epi::kFillBlocks / 4) rows = 8;
+  if (rows > 8 && blocks(rows) < (wide ? epi::kFillBlocks / 4 : 2 * epi::kFillBlocks)) rows = 8;
   const int bands = (out_size + rows - 1) / rows;
   // a column per thread; at least four waves, for the averaging and, on rows of up to 128 columns,
   // in groups that share the band's rows (one map, 83 images 64 -> 64: 8.4 us with three of four
