@@ -18,8 +18,6 @@
 namespace musc {
 namespace rscin {
 
-constexpr int kThreads = 1024;   // 16 waves share a row's n similarities
-constexpr int kWaves = kThreads / kWave;
 constexpr int kRowsAtOnce = 4;   // similarities a wave forms together
 constexpr int kSteps = 3;        // 64-vector steps whose loads are in flight together
 constexpr int kMaxN = 4096;
@@ -30,7 +28,7 @@ __device__ inline double nmax(double a, double b) { return __builtin_elementwise
 
 struct KList {
   int k[kMaxK];
-  int n;
+  int n, most;
 };
 
 // wave_sum of several values, their exchanges in flight together.
@@ -51,12 +49,15 @@ __device__ inline void wave_sums(double (&v)[kCount]) {
 // row at a time waited for memory once per 64 channels; 16 waves share the row; each
 // entry's rank is counted once for all of k_list, by several lanes.  N = 83, d = 768,
 // k = 1, 2, 3, right after the map kernel: 12.1 us, against 88.7 us with 4 waves, one
-// similarity at a time, scalar loads and a rank count per k (N = 1000: 0.50 against
-// 1.08 ms).
-template <int kVec>  // floats per load: 4 when every row is 16-byte aligned, else 1
+// similarity at a time, scalar loads and a rank count per k.  From N = 513 on the n^2
+// comparisons of a row are most of it and n rows fill the chip: 4 waves, more workgroups on
+// a CU; up to N = 16 4 waves form every similarity at once (N = 1600, d = 512:
+// 1.02 ms; 2.10 with 16 waves and both comparisons for every entry; 83 images 11.6 us).
+template <int kVec, int kThreads>  // floats per load: 4 when every row is 16-byte aligned, else 1
 __global__ __launch_bounds__(kThreads) void rscin_kernel(const float* __restrict__ x, const double* __restrict__ raw,
                                                          int n, int d, int share, KList ks, float* __restrict__ out) {
   typedef float vec __attribute__((ext_vector_type(kVec)));
+  constexpr int kWaves = kThreads / kWave;
   extern __shared__ double w[];  // n similarities of row i
   __shared__ double s_range[2][kWaves];
   __shared__ double s_part[kMaxK][2][kWaves];
@@ -131,17 +132,24 @@ __global__ __launch_bounds__(kThreads) void rscin_kernel(const float* __restrict
   for (int q = 0; q < kMaxK; ++q) num[q] = den[q] = 0.0;
   // an entry's rank is counted by `share` neighbouring lanes, each over every share-th entry
   for (int t0 = 0; t0 < n * share; t0 += kThreads) {
+    if (t0 + wave * kWave >= n * share) break;  // a wave past the last entry counts nothing
     const int j = (t0 + tid) / share, m0 = (t0 + tid) % share;
     const bool own = j < n && m0 == 0;
     const double v = w[min(j, n - 1)];
-    int rank = 0;  // entries strictly before j in descending order
+    // entries strictly before j in descending order: those above, and equal ones with a lower
+    // index; only within the wave's own entries does a comparison depend on the lane's index
+    int rank = 0, m = m0;
+    const int lowest = (t0 + wave * kWave) / share, past = min((t0 + wave * kWave + kWave - 1) / share + 1, n);
 #pragma unroll 4
-    for (int m = m0; m < n; m += share) {
+    for (; m < lowest; m += share) rank += w[m] >= v;
+    for (; m < past; m += share) {
       const double u = w[m];
       rank += (u > v) | ((u == v) & (m < j));
     }
+#pragma unroll 4
+    for (; m < n; m += share) rank += w[m] > v;
     for (int off = share / 2; off >= 1; off >>= 1) rank += __shfl_xor(rank, off, kWave);
-    if (own) {
+    if (own && rank < ks.most) {
       const double s01 = (double)(float)((raw[j] - lo) / span);
 #pragma unroll
       for (int q = 0; q < kMaxK; ++q)
@@ -193,11 +201,15 @@ extern "C" int musc_rscin_f32(const float* cls_tokens, const double* image_score
   for (int q = 0; q < n_k; ++q) {
     if (k_list[q] < 1 || k_list[q] > n) return MUSC_ERR_INVALID_ARG;
     ks.k[q] = k_list[q];
+    ks.most = ks.most > k_list[q] ? ks.most : k_list[q];
   }
+  const int threads = n <= 16 || n > 512 ? 256 : 1024;
   int share = 1;  // lanes per entry of the rank count
-  while (share < 16 && n * share * 2 <= rscin::kThreads) share *= 2;
+  while (share < 16 && n * share * 2 <= threads) share *= 2;
   const bool vec4 = d % 4 == 0 && (reinterpret_cast<uintptr_t>(cls_tokens) & 15) == 0;
-  hipLaunchKernelGGL((vec4 ? rscin::rscin_kernel<4> : rscin::rscin_kernel<1>), dim3(n), dim3(rscin::kThreads),
-                     (size_t)n * sizeof(double), stream, cls_tokens, image_scores, n, d, share, ks, out);
+  auto kernel = threads == 256 ? (vec4 ? rscin::rscin_kernel<4, 256> : rscin::rscin_kernel<1, 256>)
+                               : (vec4 ? rscin::rscin_kernel<4, 1024> : rscin::rscin_kernel<1, 1024>);
+  hipLaunchKernelGGL(kernel, dim3(n), dim3(threads), (size_t)n * sizeof(double), stream, cls_tokens, image_scores, n, d,
+                     share, ks, out);
   return check_launch();
 }

@@ -52,3 +52,25 @@ def test_row_widths_and_pool_sizes(device, n, d, offset):
         assert np.isnan(got).all()
         return
     np.testing.assert_allclose(got, orc.rscin_bruteforce_f64(raw, cls, ks), rtol=0, atol=1.2e-7)
+
+
+@pytest.mark.parametrize('n', [3, 16, 17, 64, 129, 512, 513, 700, 1024, 1030, 2100])
+def test_equal_similarities_rank_by_index(device, n):
+    # few distinct class tokens, so that whole groups of similarities are equal and every cut of
+    # k_list falls inside one: the entries with the lower indices are kept.  4-bit channels: the
+    # sums are exact in any order
+    rng = np.random.default_rng(n)
+    distinct = rng.integers(1, 5, (5, 8)).astype(np.float32)
+    cls = distinct[rng.integers(0, 5, n)]
+    raw = rng.permutation(n) / n + 0.25
+    ks = sorted({1, min(2, n), min(16, n), max(1, n // 7), n // 2 + 1, n})
+    got = RsCIN(torch.from_numpy(raw).to(device), torch.from_numpy(cls).to(device), ks).cpu().numpy()
+    w = cls.astype(np.float64) @ cls.astype(np.float64).T
+    s01 = ((raw - raw.min()) / (raw.max() - raw.min())).astype(np.float32).astype(np.float64)
+    order = np.argsort(-w, axis=1, kind='stable')
+    ref = np.zeros(n)
+    for k in ks:
+        top = order[:, :k]
+        v = np.take_along_axis(w, top, 1)
+        ref += (v * s01[top]).sum(1) / v.sum(1)
+    np.testing.assert_allclose(got, ref / len(ks), rtol=0, atol=1.2e-7)
