@@ -96,9 +96,9 @@ __global__ __launch_bounds__(kMaxThreads) void maps_kernel(const double* __restr
       int h0 = next_h0;
       double lh1 = next_lh1;
       if constexpr (kGroups > 1) {
-        const double sy = scale * (y0 + y);
-        h0 = (int)sy;
-        lh1 = sy - h0;
+        const double yy = y0 + y;
+        h0 = (int)(scale * yy);
+        lh1 = __builtin_fma(scale, yy, -(double)h0);  // rounded once, as the table's difference is
       } else {
         const int yn = min(y + 1, ye - 1);
         next_h0 = s_h0[yn];
